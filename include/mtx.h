@@ -161,7 +161,7 @@ int32_t mtx_trace_closest(mtx_handle accel, const mtx_ray *rays, uint32_t count,
  * For callers that cannot allocate device memory (code under HIP graph
  * capture, tight serving loops, harnesses that forbid hipMalloc). The
  * traversal stacks' spill slices and the work counters live in a static
- * device array of 72 MiB + 256 B (1024 persistent blocks x 128 lanes x 144
+ * device array of 72 MiB + 4 KiB (1024 persistent blocks x 128 lanes x 144
  * stack entries) that every device holds from library load until the process
  * ends; its device address is looked up once per device on the first call.
  * Same results as mtx_trace_closest, bit for bit. At most 2^30 rays per call
@@ -438,7 +438,7 @@ int32_t mtx_target_read_accumulators(mtx_handle target, double *sums, size_t cap
 typedef struct mtx_wavefront_tuning {
   uint32_t struct_size;
   uint32_t max_paths_in_flight;    /* paths per generation (0 = keep) */
-  uint32_t trace_kernel;           /* 0 one ray per thread, 1 persistent lane-refill walker */
+  uint32_t trace_kernel;           /* 0 or 1; both run the wave-scheduled traversal kernels */
   uint32_t lds_stack;              /* traversal LDS stack entries per lane: 16, 24 or 32 */
   uint32_t trace_oversubscription; /* trace grid = CUs x resident blocks x this (>= 1) */
   uint32_t shade_oversubscription; /* shade grid likewise (>= 1) */

@@ -3,7 +3,7 @@
 The reference's only tuner is the tile-size predictor of TileRender.ts
 (:302-490), which fits tile area to a time budget from GPU timestamps. Here
 the knobs are the wavefront kernels' launch shape (mtx_wavefront_tuning):
-traversal form, LDS stack depth, grid oversubscription, the shade kernel's
+LDS stack depth, grid oversubscription, the shade kernel's
 occupancy target, the queue length below which the tail kernel finishes a
 generation, and the number of paths in flight. The tuner measures each
 candidate with HIP events (RenderTarget.render_timed) on a short probe
@@ -21,7 +21,6 @@ import json
 import os
 
 SPACE = {
-    "trace_kernel": [0, 1],
     "lds_stack": [16, 24, 32],
     "trace_oversubscription": [1, 2, 4],
     "shade_waves_per_simd": [1, 2, 4],
@@ -31,7 +30,7 @@ SPACE = {
     "queue_sort": [0, 1],
     "lds_stack_closest": [0, 16, 24, 32],  # 0: the any-hit depth (lds_stack)
 }
-ORDER = ["max_paths_in_flight", "tail_paths", "queue_sort", "trace_kernel", "trace_oversubscription",
+ORDER = ["max_paths_in_flight", "tail_paths", "queue_sort", "trace_oversubscription",
          "shade_waves_per_simd", "shade_oversubscription", "lds_stack", "lds_stack_closest"]
 
 

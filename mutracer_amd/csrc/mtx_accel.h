@@ -51,8 +51,10 @@ static_assert(sizeof(InstSlot) == 128, "InstSlot");
 // stack's operations too.
 #if defined(__HIP_DEVICE_COMPILE__)
 #define MTX_AS_GLOBAL __attribute__((address_space(1)))
+#define MTX_AS_LDS __attribute__((address_space(3)))
 #else
 #define MTX_AS_GLOBAL
+#define MTX_AS_LDS
 #endif
 template <class T>
 __device__ __forceinline__ const MTX_AS_GLOBAL T *as_global(const T *p) {
@@ -150,9 +152,14 @@ constexpr int kMaxStack = 160;
 template <int kLds>
 struct LaneStackT {
   static_assert(kLds >= kMinLdsStack && kLds <= kMaxStack, "LDS stack depth");
-  int32_t *lds;
+  // Pointers with their address spaces: through generic pointers the compiler
+  // merges the two sides of get() into one flat load, which takes the vector
+  // memory path for entries that lie in LDS.
+  MTX_AS_LDS int32_t *lds;
   int32_t ldsStride;
-  int32_t *spill;
+  MTX_AS_GLOBAL int32_t *spill;
+  __device__ __forceinline__ LaneStackT(int32_t *l, int32_t stride, int32_t *s)
+      : lds((MTX_AS_LDS int32_t *)l), ldsStride(stride), spill((MTX_AS_GLOBAL int32_t *)s) {}
   __device__ __forceinline__ void put(int i, int32_t v) {
     if (i < kLds) lds[i * ldsStride] = v; else spill[i - kLds] = v;
   }

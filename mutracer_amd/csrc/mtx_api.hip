@@ -6,6 +6,7 @@
 
 #include "mtx_fetch.h"
 #include "mtx_registry.h"
+#include "mtx_walk.h"
 
 namespace mtx {
 
@@ -21,14 +22,14 @@ uint64_t Registry::next() { return nextHandle.fetch_add(1); }
 constexpr int kTraceBlock = 128;
 
 __global__ void k_zero_counters(uint32_t *__restrict__ c) {
-  if (threadIdx.x < (uint32_t)kXcds) c[threadIdx.x] = 0u;
+  if (threadIdx.x < (uint32_t)kXcds) c[threadIdx.x * kCtrStride] = 0u;
 }
 
-// Ray queries: the same traversal, occupancy targets and XCD-segmented work
-// distribution as the wavefront trace (closest hit) and shadow (any hit)
-// kernels; `ctr` holds the kXcds chunk counters, zeroed before the launch.
-template <int kMode>  // 0 closest, 1 any, 2 counters
-__global__ void __launch_bounds__(kTraceBlock, kMode == 1 ? kShadowWaves : kTraceWaves)
+// Ray queries: the traversal of the wavefront trace (closest hit) and shadow
+// (any hit) kernels over a caller's rays; `ctr` holds the queue's chunk
+// counters, zeroed before the launch.
+template <int kMode>  // 0 closest, 1 any, 2 counters, 3 closest with visit counts
+__global__ void __launch_bounds__(kTraceBlock, kMode == 1 ? kOcclusionWaves : kTraceWaves)
 k_trace(const AccelView *__restrict__ viewp, const mtx_ray *__restrict__ rays, uint32_t n,
         mtx_hit *__restrict__ hits, uint32_t *__restrict__ out, uint32_t flags, int32_t *__restrict__ spill,
         uint32_t *__restrict__ ctr) {
@@ -36,47 +37,37 @@ k_trace(const AccelView *__restrict__ viewp, const mtx_ray *__restrict__ rays, u
   const AccelView acc = *viewp;
   LaneStackT<kMinLdsStack> st{lds + threadIdx.x, kTraceBlock,
                               spill + ((size_t)blockIdx.x * kTraceBlock + threadIdx.x) * (kMaxStack - kMinLdsStack)};
-  const bool doubleSided = (flags & MTX_TRACE_DOUBLE_SIDED) != 0;
-  auto ray = [&](uint32_t i) {
+  const bool doubleSided = kMode == 1 || (flags & MTX_TRACE_DOUBLE_SIDED) != 0;
+  auto load = [&](uint32_t i, RayIn &r) {
     const float4 *r4 = reinterpret_cast<const float4 *>(rays + i);
-    float4 a = r4[0], b = r4[1];
-    f3 o{a.x, a.y, a.z}, d{b.x, b.y, b.z};
-    TraceHit h;
-    TraceCounters c{0, 0, 0};
+    const float4 a = r4[0], b = r4[1];
+    r.o = f3of(a);
+    r.d = f3of(b);
+    r.tMax = kMode == 1 ? fminf(fmaxf(a.w, 0.0f), kRayMaxDistance) : kRayMaxDistance;
+    r.curTri = r.curSlot = -1;
+    r.id = i;
+  };
+  auto covers = [](uint32_t, int32_t, int32_t, f3) { return true; };
+  auto hit = [&](uint32_t i, float t, f3 b, int32_t slot, int32_t, int32_t source) {
+    if (kMode == 2) return;
+    hits[i] = mtx_hit{1u, fint(acc.slots[slot].c2.w), source, t, {b.x, b.y, b.z}, 0u};
+  };
+  auto done = [&](uint32_t i, bool any, const TraceCounters &c) {
     if (kMode == 1) {
-      float tMax = fminf(fmaxf(a.w, 0.0f), kRayMaxDistance);
-      out[i] = traverse<true, false>(acc, o, d, tMax, true, 1, -1, -1, st, h, nullptr) ? 1u : 0u;
+      out[i] = any ? 1u : 0u;
       return;
     }
-    const bool counting = kMode == 2 || (flags & MTX_TRACE_COUNT);
-    if (counting) traverse<false, true>(acc, o, d, kRayMaxDistance, doubleSided, 0, -1, -1, st, h, &c);
-    else traverse<false, false>(acc, o, d, kRayMaxDistance, doubleSided, 0, -1, -1, st, h, nullptr);
     if (kMode == 2) {
       out[(size_t)i * 3] = c.boxes;
       out[(size_t)i * 3 + 1] = c.tris;
       out[(size_t)i * 3 + 2] = c.instances;
       return;
     }
-    mtx_hit o4;
-    o4.hit = h.hit ? 1u : 0u;
-    if (h.hit) {
-      const InstSlot &s = acc.slots[h.slot];
-      o4.instance = fint(s.c2.w);
-      o4.primitive = fint(s.tris[h.tri].v0.w);
-      o4.t = h.t;
-      o4.barycentric[0] = h.bary.x;
-      o4.barycentric[1] = h.bary.y;
-      o4.barycentric[2] = h.bary.z;
-    } else {
-      o4.instance = -1;
-      o4.primitive = -1;
-      o4.t = kRayMaxDistance;
-      o4.barycentric[0] = o4.barycentric[1] = o4.barycentric[2] = 0.0f;
-    }
-    o4.visits = counting ? c.boxes + c.tris : 0u;
-    hits[i] = o4;
+    if (!any) hits[i] = mtx_hit{0u, -1, -1, kRayMaxDistance, {0.0f, 0.0f, 0.0f}, 0u};
+    if (kMode == 3) hits[i].visits = c.boxes + c.tris;
   };
-  for_each_ray<kMode == 1 ? kShadowFetch : kTraceFetch>(n, ctr, ray);
+  trace_queue<kMode == 1, (kMode >= 2), false, false>(
+      n, ctr, acc, doubleSided, st, load, hit, covers, done);
 }
 
 // Spill slices for the traversal stacks and chunk counters of the ray
@@ -93,7 +84,7 @@ static uint32_t *counters_for(hipStream_t s) {
   MTX_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> g(gSpill.m);
   auto &b = gSpill.counters[{dev, s}];
-  if (!b) b = std::make_shared<DevBuf<uint32_t>>(kXcds);
+  if (!b) b = std::make_shared<DevBuf<uint32_t>>(kXcds * kCtrStride);
   return b->ptr;
 }
 
@@ -121,34 +112,46 @@ int32_t *spill_for(hipStream_t s, uint32_t blocksNeeded, uint32_t blockThreads) 
   return b->ptr;
 }
 
+static const void *trace_kernel(int mode) {
+  return mode == 0   ? (const void *)k_trace<0>
+         : mode == 1 ? (const void *)k_trace<1>
+         : mode == 2 ? (const void *)k_trace<2> : (const void *)k_trace<3>;
+}
+// Blocks of a query of n rays: at most `most` (a multiple of 8, one share per
+// XCD), and at most one wave per ray (short queries run with one ray or a few
+// per wave, see WorkQueue).
+static uint32_t query_grid(uint32_t n, uint32_t most) {
+  constexpr uint32_t wpb = kTraceBlock / 64;
+  return std::max<uint32_t>(8u, std::min<uint64_t>(most, ((uint64_t)n + wpb - 1) / wpb + 7) & ~7u);
+}
+static uint32_t resident_grid(int mode) {
+  static uint32_t bpc[4] = {0, 0, 0, 0};
+  if (!bpc[mode]) {
+    int b = 0;
+    MTX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, trace_kernel(mode), kTraceBlock, 0));
+    bpc[mode] = (uint32_t)std::max(1, b);
+  }
+  return trace_grid() / 8u * bpc[mode];
+}
+static void launch_query(int mode, uint32_t grid, const Accel &A, const mtx_ray *rays, uint32_t n, mtx_hit *hits,
+                         uint32_t *out, uint32_t flags, int32_t *spill, uint32_t *ctr, hipStream_t s) {
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, ctr);
+  switch (mode) {
+    case 0: hipLaunchKernelGGL(k_trace<0>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill, ctr); break;
+    case 1: hipLaunchKernelGGL(k_trace<1>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill, ctr); break;
+    case 2: hipLaunchKernelGGL(k_trace<2>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill, ctr); break;
+    default: hipLaunchKernelGGL(k_trace<3>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill, ctr); break;
+  }
+  MTX_HIP(hipGetLastError());
+}
+
 static void launch_trace(int mode, const Accel &A, const mtx_ray *rays, uint32_t n, mtx_hit *hits, uint32_t *out,
                          uint32_t flags, hipStream_t s) {
   MTX_REQUIRE(A.max_stack() <= (uint32_t)kMaxStack, MTX_INVALID_STATE, "scene deeper than the traversal stack");
   if (!n) return;
-  // Persistent grid: the resident blocks of the kernel on every CU.
-  static uint32_t bpc[3] = {0, 0, 0};
-  const void *k = mode == 0 ? (const void *)k_trace<0> : mode == 1 ? (const void *)k_trace<1> : (const void *)k_trace<2>;
-  if (!bpc[mode]) {
-    int b = 0;
-    MTX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k, kTraceBlock, 0));
-    bpc[mode] = (uint32_t)std::max(1, b);
-  }
-  uint32_t grid = trace_grid() / 8u * bpc[mode];
-  uint32_t rayBlocks = (n + kTraceBlock - 1) / kTraceBlock;
-  grid = std::min<uint32_t>(grid, ((rayBlocks + 7u) / 8u) * 8u);
-  int32_t *spill = spill_for(s, grid, kTraceBlock);
-  uint32_t *ctr = counters_for(s);
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, ctr);
-  if (mode == 0)
-    hipLaunchKernelGGL(k_trace<0>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill,
-                       ctr);
-  else if (mode == 1)
-    hipLaunchKernelGGL(k_trace<1>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill,
-                       ctr);
-  else
-    hipLaunchKernelGGL(k_trace<2>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, out, flags, spill,
-                       ctr);
-  MTX_HIP(hipGetLastError());
+  if (mode == 0 && (flags & MTX_TRACE_COUNT)) mode = 3;
+  const uint32_t grid = query_grid(n, resident_grid(mode));
+  launch_query(mode, grid, A, rays, n, hits, out, flags, spill_for(s, grid, kTraceBlock), counters_for(s), s);
 }
 
 // ----------------------------------------------- allocation-free ray query
@@ -158,7 +161,7 @@ static void launch_trace(int mode, const Accel &A, const mtx_ray *rays, uint32_t
 // from module load until the process ends, and nothing is allocated per call.
 constexpr uint32_t kNoAllocBlocks = 1024;
 constexpr size_t kNoAllocSpillInts = (size_t)kNoAllocBlocks * kTraceBlock * (kMaxStack - kMinLdsStack);
-constexpr size_t kNoAllocScratchBytes = kNoAllocSpillInts * sizeof(int32_t) + 256;  // + kXcds chunk counters
+constexpr size_t kNoAllocScratchBytes = kNoAllocSpillInts * sizeof(int32_t) + kXcds * kCtrStride * sizeof(uint32_t);
 constexpr uint32_t kNoAllocMaxRays = 1u << 30;
 static __device__ __align__(256) uint8_t scratch[kNoAllocScratchBytes];
 
@@ -188,20 +191,9 @@ static void launch_trace_noalloc(const Accel &A, const mtx_ray *rays, uint32_t n
   if (!n) return;
   int32_t *spill = reinterpret_cast<int32_t *>(base);
   uint32_t *ctr = reinterpret_cast<uint32_t *>(base + kNoAllocSpillInts * sizeof(int32_t));
-  static uint32_t bpc = 0;
-  if (!bpc) {
-    int b = 0;
-    MTX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, (const void *)k_trace<0>, kTraceBlock, 0));
-    bpc = (uint32_t)std::max(1, b);
-  }
-  uint32_t grid = std::min<uint32_t>(trace_grid() / 8u * bpc, kNoAllocBlocks);
-  const uint32_t rayBlocks = (n + kTraceBlock - 1) / kTraceBlock;
-  grid = std::min<uint32_t>(grid, ((rayBlocks + 7u) / 8u) * 8u);
-  grid = std::max<uint32_t>(8u, grid & ~7u);
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, ctr);
-  hipLaunchKernelGGL(k_trace<0>, dim3(grid), dim3(kTraceBlock), 0, s, A.view.ptr, rays, n, hits, nullptr, flags, spill,
-                     ctr);
-  MTX_HIP(hipGetLastError());
+  const int mode = (flags & MTX_TRACE_COUNT) ? 3 : 0;
+  const uint32_t grid = query_grid(n, std::min<uint32_t>(resident_grid(mode), kNoAllocBlocks));
+  launch_query(mode, grid, A, rays, n, hits, nullptr, flags, spill, ctr, s);
 }
 
 }  // namespace mtx

@@ -11,76 +11,99 @@ __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 constexpr int kXcds = 8;
 
 // Occupancy the register allocator must reach for the traversal kernels
-// (waves per SIMD). Measured on the 1M-triangle 1080p workload: closest-hit
-// is fastest at 6 (80 VGPRs, a few spilled; 5 unconstrained, 8 spills too
-// much), any-hit at 8 (64 VGPRs); re-measured with the unified closest-hit
-// node step, 5 and 7 are slightly slower. The 16-entry LDS stack keeps LDS
-// from capping these.
-constexpr int kTraceWaves = 6;
-constexpr int kShadowWaves = 8;
+// (waves per SIMD): 5 (96 VGPRs) for the wavefront kernels and closest-hit
+// queries, where 6 spills (closest hit of the 1M-triangle 1080p step 66.5 ms
+// against 50.2, 4 waves 62 ms; shadow rays 26.1 against 25.8), 6 (no spill)
+// for the smaller any-hit query (1.01 ms against 1.04 for 1.5M rays).
+constexpr int kTraceWaves = 5;
+constexpr int kOcclusionWaves = 6;
 
+// Idle lanes a wave gathers before it takes new rays: loading a ray and
+// writing a result cost about a hundred instructions whatever the number of
+// lanes. 8, 16 and 24 measure within 1%.
+constexpr int kRefill = 16;
 
-// Work distribution of the traversal kernels. The queue of n entries is cut
-// into kXcds contiguous segments, one per XCD (workgroups are dispatched
-// to the XCDs round-robin, so block b runs on XCD b % 8). Neighbouring queue
-// entries are spatially coherent rays (neighbouring pixels of pixel-major
-// paths, or a caller's ordered batch), so each XCD's L2 serves a small part
-// of the scene at a time.
-//   mode 0: grid-stride loop over the whole queue (no segments)
-//   mode 1: a wave takes the next kFetchChunk entries of its XCD's segment
-//           with one atomic and helps the other segments once its own is
-//           drained
-//   mode 2: static segments, each XCD's blocks stride over their own
-// Measured on the 1M-triangle 1080p workload: closest-hit is fastest with
-// mode 1 (its rays are long enough to amortize the atomic), any-hit with
-// mode 0; mode 2 loses to load imbalance, chunks above 64 serialize the
-// short queues of late events.
-constexpr int kTraceFetch = 1;
-constexpr int kShadowFetch = 0;
-constexpr uint32_t kFetchChunk = 64;
-__device__ __forceinline__ bool fetch_chunk(uint32_t *ctr, uint32_t n, uint32_t &seg, uint32_t &base,
-                                            uint32_t &limit) {
-  uint32_t b0 = 0, l0 = 0, s0 = seg;
-  if (lane_id() == 0) {
-    for (uint32_t k = 0; k < (uint32_t)kXcds; k++) {
-      const uint32_t x = (seg + k) % (uint32_t)kXcds;
-      const uint32_t b = (uint32_t)(((uint64_t)n * x) / kXcds);
-      const uint32_t e = (uint32_t)(((uint64_t)n * (x + 1)) / kXcds);
-      if (b >= e) continue;
-      const uint32_t c = atomicAdd(ctr + x, 1u);
-      if (c < (e - b + kFetchChunk - 1u) / kFetchChunk) {
-        b0 = b + c * kFetchChunk;
-        l0 = min(e, b0 + kFetchChunk);
-        s0 = x;
-        break;
+// Words between the chunk counters of two XCDs: each counter on lines of its
+// own, so that an atomic moves no line between XCDs.
+constexpr uint32_t kCtrStride = 128;
+
+// A wave's view of a queue of n entries that all waves of the grid empty
+// together. The queue is cut into chunks, the chunks into one contiguous
+// segment per XCD (block b runs on XCD b % 8), and every wave starts with a
+// chunk of its own, found without any atomic; the chunks beyond those are
+// handed out by the segment's counter, and a wave whose segment is empty
+// helps the others. A queue too short to give every lane of the grid an
+// entry is spread over the waves: each works with fewer lanes, so that rays
+// that would wait for one another in one wave run in several (4096 rays over
+// 4096 waves 160 us, three to a wave 198 us).
+// With the counters on one line, an atomic per 64 rays and eight more for
+// every wave's end, the 1.6M closest-hit rays of a 256 x 256 x 8 Cornell
+// generation took 2.27 ms; with this queue and trace_queue 0.62 ms.
+struct WorkQueue {
+  uint32_t n, chunk, chunks;
+  uint32_t *ctr;
+  uint32_t seg, base, limit;
+  int lanes, refillMin;
+  uint64_t laneMask;
+  bool open;  // chunks may be left beyond the current one
+
+  __device__ __forceinline__ uint32_t seg_lo(uint32_t x) const { return (uint32_t)(((uint64_t)chunks * x) / kXcds); }
+  __device__ __forceinline__ uint32_t seg_waves(uint32_t x) const {
+    return ((gridDim.x + (uint32_t)kXcds - 1u - x) / (uint32_t)kXcds) * (blockDim.x >> 6);
+  }
+  __device__ __forceinline__ bool set(uint32_t c) {
+    base = c * chunk;
+    limit = n - base < chunk ? n : base + chunk;
+    return true;
+  }
+
+  __device__ __forceinline__ WorkQueue(uint32_t n_, uint32_t *ctr_) : n(n_), ctr(ctr_) {
+    const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+    const uint32_t per = (uint32_t)(((uint64_t)n + waves - 1u) / waves);
+    lanes = (int)min(64u, max(1u, per));
+    chunk = lanes < 64 ? (uint32_t)lanes : 64u * min(4u, max(1u, n / (waves * 512u)));
+    chunks = (n + chunk - 1u) / chunk;
+    laneMask = lanes == 64 ? ~0ull : (1ull << lanes) - 1ull;
+    refillMin = min(lanes, kRefill);
+    seg = blockIdx.x % (uint32_t)kXcds;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t c = seg_lo(seg) + (blockIdx.x / (uint32_t)kXcds) * (blockDim.x >> 6) + wave;
+    base = limit = 0;
+    open = true;
+    if (c < seg_lo(seg + 1u)) set(c);
+  }
+
+  // Entries left for this wave (fetches a chunk when the current one is used up).
+  __device__ __forceinline__ bool more() {
+    if (base < limit) return true;
+    while (open) {
+      uint32_t first = seg_lo(seg) + seg_waves(seg), end = seg_lo(seg + 1u);
+      if (first < end) {
+        uint32_t c = 0;
+        if (lane_id() == 0) c = atomicAdd(ctr + seg * kCtrStride, 1u);
+        c = first + __builtin_amdgcn_readfirstlane(c);
+        if (c < end) return set(c);
       }
+      // This segment is empty: look for another that is not.
+      const uint32_t x = (seg + lane_id()) % (uint32_t)kXcds;
+      bool left = false;
+      if (lane_id() < (uint32_t)kXcds) {
+        const uint32_t f = seg_lo(x) + seg_waves(x), e = seg_lo(x + 1u);
+        left = f < e && f + __hip_atomic_load(ctr + x * kCtrStride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < e;
+      }
+      const uint64_t m = __ballot(left);
+      open = m != 0ull;
+      if (open) seg = (seg + (uint32_t)__builtin_ctzll(m)) % (uint32_t)kXcds;
     }
+    return false;
   }
-  base = __shfl(b0, 0);
-  limit = __shfl(l0, 0);
-  seg = __shfl(s0, 0);
-  return base < limit;
-}
-
-// Calls ray(i) once for every queue entry i < n, spread over the grid by kFetchMode.
-template <int kFetchMode, class F>
-__device__ __forceinline__ void for_each_ray(uint32_t n, uint32_t *ctr, F &&ray) {
-  if (kFetchMode == 1) {
-    // Waves beyond one per chunk could only probe drained segments: they
-    // leave at once (the first ceil(n / 64) waves keep fetching until every
-    // segment is drained, so no chunk is left behind).
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-    if (wave >= (n + kFetchChunk - 1u) / kFetchChunk) return;
-    uint32_t seg = blockIdx.x % (uint32_t)kXcds, base, limit;
-    while (fetch_chunk(ctr, n, seg, base, limit))
-      for (uint32_t i = base + lane_id(); i < limit; i += 64u) ray(i);
-  } else if (kFetchMode == 2 && gridDim.x % (uint32_t)kXcds == 0u) {
-    const uint32_t x = blockIdx.x % (uint32_t)kXcds, nb = gridDim.x / (uint32_t)kXcds;
-    const uint32_t b = (uint32_t)(((uint64_t)n * x) / kXcds), e = (uint32_t)(((uint64_t)n * (x + 1)) / kXcds);
-    for (uint32_t i = b + (blockIdx.x / kXcds) * blockDim.x + threadIdx.x; i < e; i += nb * blockDim.x) ray(i);
-  } else {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) ray(i);
+  // Hands out up to `want` entries from `first` on.
+  __device__ __forceinline__ uint32_t take(uint32_t want, uint32_t &first) {
+    const uint32_t k = min(want, limit - base);
+    first = base;
+    base += k;
+    return k;
   }
-}
+};
 
 }  // namespace mtx

@@ -98,17 +98,17 @@ struct TargetObj;
 //   qA/qB path-id queues of even/odd events
 //   s0..s3 shadow queue: (origin, tMax), (direction, path id), (payload, tri), slot
 //   counts[e] = length of event e's queue, counts[kWfShadowBase + e] = its shadow queue,
-//   counts[kWfFetchBase + 2e (+1)] = next entry the persistent trace (shadow) kernel takes
-//   counts[kWfXcdBase + (2e (+1)) * 8 + x] = next 64-entry chunk of XCD x's segment of
-//                                           event e's (shadow) queue
+//   counts[kWfXcdBase + x * kWfCtrStride + 2e (+1)] = next chunk handed out of XCD x's
+//                                           segment of event e's (shadow) queue
 //   counts[kWfTailFlag] = 1 + the event at which the tail kernel took over the
 //                         generation's remaining paths (0 while it has not)
 constexpr int kWfMaxEvents = 51;
 constexpr int kWfShadowBase = kWfMaxEvents + 1;
-constexpr int kWfFetchBase = kWfShadowBase + kWfMaxEvents + 1;
-constexpr int kWfXcdBase = kWfFetchBase + 2 * (kWfMaxEvents + 1);
+constexpr int kWfXcdBase = (kWfShadowBase + kWfMaxEvents + 1 + 127) / 128 * 128;
 constexpr int kWfXcds = 8;  // XCDs of an MI355X (counter segments per queue)
-constexpr int kWfTailFlag = kWfXcdBase + 2 * (kWfMaxEvents + 1) * kWfXcds;
+constexpr int kWfCtrStride = 128;  // words of one XCD's counters, on lines of their own
+static_assert(2 * (kWfMaxEvents + 1) <= kWfCtrStride, "counters of one XCD");
+constexpr int kWfTailFlag = kWfXcdBase + kWfCtrStride * kWfXcds;
 // Queue sorting: the shade kernel appends each continuing path to the bin of
 // its ray direction's octant, counts[kWfSortBase + kWfSortBins * e + o]
 // entries for queue e, and a gather kernel concatenates the bins into the
@@ -173,8 +173,8 @@ struct WfConfig {
   uint32_t maxPaths = 1u << 25;  // paths in flight per generation
   int traceOversub = 1;          // trace/shadow grid = CUs * resident blocks * this
   int shadeOversub = 1;
-  bool walker = false;           // persistent lane-refill traversal (else one ray per thread)
-  int ldsStack = 16;             // LDS stack entries per lane of the any-hit (and walker) kernels (16, 24 or 32)
+  uint32_t traceKernel = 0;      // mtx_wavefront_tuning.trace_kernel as set; both values run the same kernels
+  int ldsStack = 16;             // LDS stack entries per lane of the any-hit kernels (16, 24 or 32)
   int ldsStackClosest = 0;       // the same for the closest-hit trace kernel (0 = ldsStack)
   int shadeWaves = 2;            // occupancy target of the shade kernel (1..4 waves per SIMD)
   bool graphs = true;            // capture each generation's launch sequence into a hipGraph and replay it

@@ -929,7 +929,7 @@ int32_t mtx_target_set_tuning(mtx_handle target, const mtx_wavefront_tuning *t) 
   std::unique_lock<std::mutex> lk(T->busy, std::try_to_lock);
   if (!lk.owns_lock()) return MTX_BUSY;
   if (t->max_paths_in_flight) T->wfConfig.maxPaths = t->max_paths_in_flight;
-  T->wfConfig.walker = t->trace_kernel == 1;
+  T->wfConfig.traceKernel = t->trace_kernel;
   T->wfConfig.ldsStack = (int)t->lds_stack;
   T->wfConfig.traceOversub = (int)t->trace_oversubscription;
   T->wfConfig.shadeOversub = (int)t->shade_oversubscription;
@@ -949,7 +949,7 @@ int32_t mtx_target_get_tuning(mtx_handle target, mtx_wavefront_tuning *t) {
   auto T = get_target(target);
   t->struct_size = sizeof(mtx_wavefront_tuning);
   t->max_paths_in_flight = T->wfConfig.maxPaths;
-  t->trace_kernel = T->wfConfig.walker ? 1u : 0u;
+  t->trace_kernel = T->wfConfig.traceKernel;
   t->lds_stack = (uint32_t)T->wfConfig.ldsStack;
   t->trace_oversubscription = (uint32_t)T->wfConfig.traceOversub;
   t->shade_oversubscription = (uint32_t)T->wfConfig.shadeOversub;

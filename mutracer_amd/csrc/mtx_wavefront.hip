@@ -157,29 +157,37 @@ k_wf_trace(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spill
                       spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
   const uint32_t *q = queue_of(W, event);
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
-  TraceCounters tc{0u, 0u, 0u};
-  uint32_t hits = 0;
   AccelView one{};
   if (!kMulti) one = *L.one.scene.accel;
-  auto ray = [&](uint32_t i) {
+  uint64_t boxes = 0, tris = 0, instances = 0, hits = 0;
+  auto load = [&](uint32_t i, RayIn &r) {
     const uint32_t p = q[i];
-    const float4 o = W.o[p], d = W.d[p];
-    const int32_t curTri = fint(W.beta[p].w), curSlot = fint(W.alb[p].w);
-    TraceHit h;
-    if (kMulti) {
-      const AccelView av = *job_of<true>(L, W, p).scene.accel;
-      traverse<false, kCount>(av, f3of(o), f3of(d), kRayMaxDistance, event != 0, 1, curTri, curSlot, st, h, &tc);
-    } else {
-      traverse<false, kCount>(one, f3of(o), f3of(d), kRayMaxDistance, event != 0, 1, curTri, curSlot, st, h, &tc);
-    }
-    W.hitA[p] = make_float4(h.t, h.bary.x, h.bary.y, h.bary.z);
-    W.hitB[p] = make_int2(h.hit ? h.slot : -1, h.tri);
-    if (kCount) hits += h.hit ? 1u : 0u;
+    r.o = f3of(W.o[p]);
+    r.d = f3of(W.d[p]);
+    r.tMax = kRayMaxDistance;
+    r.curTri = fint(W.beta[p].w);
+    r.curSlot = fint(W.alb[p].w);
+    if (kMulti) r.acc = job_of<true>(L, W, p).scene.accel;
+    r.id = p;
   };
-  for_each_ray<kTraceFetch>(n, W.counts + kWfXcdBase + (2 * event) * kWfXcds, ray);
+  auto hit = [&](uint32_t p, float t, f3 b, int32_t slot, int32_t tri, int32_t) {
+    W.hitA[p] = make_float4(t, b.x, b.y, b.z);
+    W.hitB[p] = make_int2(slot, tri);
+  };
+  auto covers = [](uint32_t, int32_t, int32_t, f3) { return true; };
+  auto done = [&](uint32_t p, bool any, const TraceCounters &c) {
+    if (!any) W.hitB[p] = make_int2(-1, -1);
+    if (kCount) {
+      boxes += c.boxes;
+      tris += c.tris;
+      instances += c.instances;
+      hits += any ? 1u : 0u;
+    }
+  };
+  trace_queue<false, kCount, kMulti, false>(n, W.counts + kWfXcdBase + 2 * event, one, event != 0, st, load, hit,
+                                            covers, done);
   if (kCount) {
-    const uint64_t v[5] = {(blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u, tc.boxes, tc.tris, tc.instances,
-                           hits};
+    const uint64_t v[5] = {(blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u, boxes, tris, instances, hits};
     const int slots[5] = {kWorkClosestRays, kWorkBoxes, kWorkTris, kWorkInstances, kWorkHits};
     flush_work(L.work, v, slots);
   }
@@ -295,7 +303,7 @@ __device__ __forceinline__ void add_payload(const WfBuffers &W, uint32_t p, floa
 }
 
 template <bool kMulti, bool kCount, int kLds, bool kAlpha>
-__global__ void __launch_bounds__(kWfTraceBlock, kShadowWaves)
+__global__ void __launch_bounds__(kWfTraceBlock, kTraceWaves)
 k_wf_shadow(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spill) {
   __shared__ int32_t lds[kLds * kWfTraceBlock];
   const uint32_t n = W.counts[kWfShadowBase + event];
@@ -303,28 +311,40 @@ k_wf_shadow(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spil
   LaneStackT<kLds> st{lds + threadIdx.x, kWfTraceBlock,
                       spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
-  TraceCounters tc{0u, 0u, 0u};
   AccelView one{};
   if (!kMulti) one = *L.one.scene.accel;
-  auto ray = [&](uint32_t i) {
-    const float4 a = W.s0[i], b = W.s1[i], c = W.s2[i];
-    const uint32_t p = (uint32_t)fint(b.w);
-    TraceHit h;
-    bool occluded;
-    if (kMulti) {
-      const GpuScene &S = job_of<true>(L, W, p).scene;
-      const AccelView av = *S.accel;
-      occluded = traverse<true, kCount>(av, f3of(a), f3of(b), a.w, true, 1, fint(c.w), W.s3[i], st, h, &tc,
-                                        coverage<kAlpha>(&S));
-    } else {
-      occluded = traverse<true, kCount>(one, f3of(a), f3of(b), a.w, true, 1, fint(c.w), W.s3[i], st, h, &tc,
-                                        coverage<kAlpha>(&L.one.scene));
-    }
-    if (!occluded) add_payload(W, p, c);
+  uint64_t boxes = 0, tris = 0, instances = 0;
+  auto path = [&](uint32_t i) { return (uint32_t)fint(W.s1[i].w); };
+  auto load = [&](uint32_t i, RayIn &r) {
+    const float4 a = W.s0[i], b = W.s1[i];
+    r.o = f3of(a);
+    r.d = f3of(b);
+    r.tMax = a.w;
+    r.curTri = fint(W.s2[i].w);
+    r.curSlot = W.s3[i];
+    if (kMulti) r.acc = job_of<true>(L, W, (uint32_t)fint(b.w)).scene.accel;
+    r.id = i;
   };
-  for_each_ray<kShadowFetch>(n, W.counts + kWfXcdBase + (2 * event + 1) * kWfXcds, ray);
+  auto hit = [](uint32_t, float, f3, int32_t, int32_t, int32_t) {};
+  auto covers = [&](uint32_t i, int32_t slot, int32_t tri, f3 b) {
+    if constexpr (kAlpha) {
+      return alpha_covers(kMulti ? job_of<true>(L, W, path(i)).scene : L.one.scene, slot, tri, b);
+    } else {
+      return true;
+    }
+  };
+  auto done = [&](uint32_t i, bool any, const TraceCounters &c) {
+    if (!any) add_payload(W, path(i), W.s2[i]);
+    if (kCount) {
+      boxes += c.boxes;
+      tris += c.tris;
+      instances += c.instances;
+    }
+  };
+  trace_queue<true, kCount, kMulti, kAlpha>(n, W.counts + kWfXcdBase + 2 * event + 1, one, true, st, load, hit, covers,
+                                            done);
   if (kCount) {
-    const uint64_t v[4] = {tc.boxes, tc.tris, tc.instances, (blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u};
+    const uint64_t v[4] = {boxes, tris, instances, (blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u};
     const int slots[4] = {kWorkShadowBoxes, kWorkShadowTris, kWorkShadowInstances, kWorkShadowRays};
     flush_work(L.work, v, slots);
   }
@@ -398,86 +418,6 @@ k_wf_tail(const WfLaunch L, WfBuffers W, int event, uint32_t tailPaths, int32_t 
 #pragma unroll
     for (int k = 0; k < 9; k++) slots[k] = kWorkTailBase + k;
     flush_work(L.work, v, slots);
-  }
-}
-
-// Persistent closest-hit / any-hit kernels over Walker: each lane takes a
-// new queue entry (wave-aggregated atomic on counts[kWfFetchBase + 2e (+1)])
-// as soon as its previous ray has finished.
-template <bool kMulti, bool kShadow, bool kCount, int kLds, bool kAlpha>
-__global__ void __launch_bounds__(kWfTraceBlock)
-k_wf_walk(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spill) {
-  __shared__ int32_t lds[kLds * kWfTraceBlock];
-  const uint32_t n = W.counts[kShadow ? kWfShadowBase + event : event];
-  if (n == 0u || W.counts[kWfTailFlag]) return;
-  uint32_t *fetch = W.counts + kWfFetchBase + 2 * event + (kShadow ? 1 : 0);
-  WalkStack<kLds> st{lds + threadIdx.x, kWfTraceBlock,
-                     spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
-  const uint32_t *q = queue_of(W, event);
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
-  AccelView av{};
-  const GpuScene *scene = &L.one.scene;  // the scene of the lane's ray (coverage of masked instances)
-  if (!kMulti) av = *L.one.scene.accel;
-  Walker<kShadow, kCount> w;
-  bool have = false, exhausted = false;
-  uint32_t entry = 0, path = 0;
-  uint64_t totals[4] = {0, 0, 0, 0};
-  const bool doubleSided = kShadow ? true : event != 0;
-  const int bounces = 1;  // closest hit: depth-0 paths store slot -1 (store_path)
-  while (true) {
-    const bool need = !have && !exhausted;
-    const uint32_t idx = wave_append(fetch, need);
-    if (need) {
-      if (idx < n) {
-        entry = idx;
-        if (kShadow) {
-          const float4 a = W.s0[idx], b = W.s1[idx], c = W.s2[idx];
-          path = (uint32_t)fint(b.w);
-          if (kMulti) {
-            scene = &job_of<true>(L, W, path).scene;
-            av = *scene->accel;
-          }
-          w.init(av, f3of(a), f3of(b), a.w, doubleSided, bounces, fint(c.w), W.s3[idx], st);
-        } else {
-          path = q[idx];
-          if (kMulti) av = *job_of<true>(L, W, path).scene.accel;
-          const float4 o = W.o[path], d = W.d[path];
-          w.init(av, f3of(o), f3of(d), kRayMaxDistance, doubleSided, bounces, fint(W.beta[path].w),
-                 fint(W.alb[path].w), st);
-        }
-        have = true;
-      } else {
-        exhausted = true;
-      }
-    }
-    if (!__any(have)) break;
-    if (have && (w.done || w.step(av, st, coverage<kAlpha>(scene)))) {
-      have = false;
-      if (kShadow) {
-        if (!w.hit) add_payload(W, path, W.s2[entry]);
-      } else {
-        W.hitA[path] = make_float4(w.t, w.bary.x, w.bary.y, w.bary.z);
-        W.hitB[path] = make_int2(w.hit ? w.hitSlot : -1, w.hitTri);
-      }
-      if (kCount) {
-        totals[0] += w.cnt.boxes;
-        totals[1] += w.cnt.tris;
-        totals[2] += w.cnt.instances;
-        totals[3] += (!kShadow && w.hit) ? 1u : 0u;
-      }
-    }
-  }
-  if (kCount) {
-    const uint64_t first = (blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u;
-    if (kShadow) {
-      const uint64_t v[4] = {totals[0], totals[1], totals[2], first};
-      const int slots[4] = {kWorkShadowBoxes, kWorkShadowTris, kWorkShadowInstances, kWorkShadowRays};
-      flush_work(L.work, v, slots);
-    } else {
-      const uint64_t v[5] = {first, totals[0], totals[1], totals[2], totals[3]};
-      const int slots[5] = {kWorkClosestRays, kWorkBoxes, kWorkTris, kWorkInstances, kWorkHits};
-      flush_work(L.work, v, slots);
-    }
   }
 }
 
@@ -637,32 +577,6 @@ WfBuffers WfBuffers::Owner::view(uint32_t nPaths, bool sort) const {
 }
 
 template <bool kMulti, bool kShadow, int kLds>
-static void launch_walk_lds(uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W, int e,
-                            int32_t *spill) {
-  if (kShadow && L.masked) {
-    if (L.work)
-      hipLaunchKernelGGL((k_wf_walk<kMulti, kShadow, true, kLds, true>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                         spill);
-    else
-      hipLaunchKernelGGL((k_wf_walk<kMulti, kShadow, false, kLds, true>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W,
-                         e, spill);
-  } else if (L.work) {
-    hipLaunchKernelGGL((k_wf_walk<kMulti, kShadow, true, kLds, false>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                       spill);
-  } else {
-    hipLaunchKernelGGL((k_wf_walk<kMulti, kShadow, false, kLds, false>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W,
-                       e, spill);
-  }
-}
-template <bool kMulti, bool kShadow>
-static void launch_walk(const WfConfig &cfg, uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W,
-                        int e, int32_t *spill) {
-  if (cfg.ldsStack <= 16) launch_walk_lds<kMulti, kShadow, 16>(grid, s, L, W, e, spill);
-  else if (cfg.ldsStack <= 24) launch_walk_lds<kMulti, kShadow, 24>(grid, s, L, W, e, spill);
-  else launch_walk_lds<kMulti, kShadow, 32>(grid, s, L, W, e, spill);
-}
-
-template <bool kMulti, bool kShadow, int kLds>
 static void launch_trace_lds(uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W, int e,
                              int32_t *spill) {
   if (kShadow) {
@@ -698,11 +612,10 @@ static void launch_trace(const WfConfig &cfg, uint32_t grid, hipStream_t s, cons
 }
 
 struct Grids {
-  uint32_t trace, shadow, walk, shade, tail, cus;
+  uint32_t trace, shadow, shade, tail, cus;
 };
 static Grids grids_for(const WfConfig &cfg) {
-  static int closestBpc[3] = {0, 0, 0}, shadowBpc[3] = {0, 0, 0}, shadeBpc[5] = {0, 0, 0, 0, 0},
-             walkBpc[3] = {0, 0, 0}, tailBpc = 0;
+  static int closestBpc[3] = {0, 0, 0}, shadowBpc[3] = {0, 0, 0}, shadeBpc[5] = {0, 0, 0, 0, 0}, tailBpc = 0;
   const int cus = cu_count();
   auto level = [](int d) { return d <= 16 ? 0 : (d <= 24 ? 1 : 2); };
   const int li = level(cfg.ldsStack), lc = level(cfg.ldsStackClosest ? cfg.ldsStackClosest : cfg.ldsStack);
@@ -724,19 +637,12 @@ static Grids grids_for(const WfConfig &cfg) {
                   : sw == 3 ? (const void *)k_wf_shade<false, 3, true> : (const void *)k_wf_shade<false, 4, true>;
     shadeBpc[sw] = blocks_per_cu(k, kWfShadeBlock, 0);
   }
-  if (!walkBpc[li]) {
-    const void *k = li == 0 ? (const void *)k_wf_walk<false, false, false, 16, false>
-                  : li == 1 ? (const void *)k_wf_walk<false, false, false, 24, false>
-                            : (const void *)k_wf_walk<false, false, false, 32, false>;
-    walkBpc[li] = blocks_per_cu(k, kWfTraceBlock, 0);
-  }
   if (!tailBpc) tailBpc = blocks_per_cu((const void *)k_wf_tail<false, false, true, false>, kWfShadeBlock, 0);
   Grids g;
   g.cus = (uint32_t)cus;
   g.tail = (uint32_t)(cus * tailBpc);
   g.trace = (uint32_t)(cus * closestBpc[lc] * std::max(1, cfg.traceOversub));
   g.shadow = (uint32_t)(cus * shadowBpc[li] * std::max(1, cfg.traceOversub));
-  g.walk = (uint32_t)(cus * walkBpc[li] * std::max(1, cfg.traceOversub));
   g.shade = (uint32_t)(cus * shadeBpc[sw] * std::max(1, cfg.shadeOversub));
   return g;
 }
@@ -792,10 +698,7 @@ static void run_generation(const WfLaunch &L, const WfBuffers &W, int eventLimit
       te();
     }
     tb(1);
-    if (cfg.walker)
-      launch_walk<kMulti, false>(cfg, g.walk, s, L, W, e, spill);
-    else
-      launch_trace<kMulti, false>(cfg, g.trace, s, L, W, e, spill);
+    launch_trace<kMulti, false>(cfg, g.trace, s, L, W, e, spill);
     te();
     tb(2);
     if (full) launch_shade<kMulti, true>(cfg, g, s, L, W, e);
@@ -803,10 +706,7 @@ static void run_generation(const WfLaunch &L, const WfBuffers &W, int eventLimit
     if (W.qSort && e < eventLimit) hipLaunchKernelGGL(k_wf_gather, dim3(genGrid), dim3(256), 0, s, W, e + 1);
     te();
     tb(3);
-    if (cfg.walker)
-      launch_walk<kMulti, true>(cfg, g.walk, s, L, W, e, spill);
-    else
-      launch_trace<kMulti, true>(cfg, g.shadow, s, L, W, e, spill);
+    launch_trace<kMulti, true>(cfg, g.shadow, s, L, W, e, spill);
     te();
   }
   const uint32_t accGrid = std::min<uint32_t>((pixels + 255) / 256, g.cus * 16u);
@@ -854,7 +754,7 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
   const uint32_t maxPaths = std::max<uint32_t>(cfg.maxPaths, p0.pixelCount);
   const uint32_t genMax = std::max<uint32_t>(1u, maxPaths / p0.pixelCount);
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(std::max(std::max(g.trace, g.shadow), g.walk), g.tail), kWfTraceBlock);
+  int32_t *spill = spill_for(s, std::max(std::max(g.trace, g.shadow), g.tail), kWfTraceBlock);
   const int eventLimit = std::min((int)p0.bounces * 3, 50);
   uint32_t done = 0;
   while (done < p0.samples) {
@@ -893,7 +793,7 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
       key = fnv(key, ptrs, sizeof ptrs);
       key = fnv(key, &L.one.acc.pixels, sizeof L.one.acc.pixels);
       key = fnv(key, &W.nPaths, sizeof W.nPaths);
-      const int64_t cf[10] = {cfg.maxPaths, cfg.traceOversub, cfg.shadeOversub, cfg.walker, cfg.ldsStack,
+      const int64_t cf[9] = {cfg.maxPaths, cfg.traceOversub, cfg.shadeOversub, cfg.ldsStack,
                               cfg.shadeWaves, cfg.graphs, cfg.tailPaths, cfg.queueSort, cfg.ldsStackClosest};
       key = fnv(key, cf, sizeof cf);
       key = fnv(key, &spill, sizeof spill);
@@ -926,7 +826,7 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
   if (!nJobs || !nPaths) return;
   MTX_REQUIRE(nJobs <= kMaxJobsPerRound, MTX_INVALID_ARGUMENT, "too many jobs in one round");
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(std::max(std::max(g.trace, g.shadow), g.walk), g.tail), kWfTraceBlock);
+  int32_t *spill = spill_for(s, std::max(std::max(g.trace, g.shadow), g.tail), kWfTraceBlock);
   buf.ensure(nPaths, cfg.queueSort);
   const WfBuffers W = buf.view(nPaths, cfg.queueSort);
   WfLaunch L;
@@ -950,7 +850,7 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
     key = fnv(key, &L, sizeof L);
     const void *ptrs[4] = {W.o, W.counts, W.rng, spill};
     key = fnv(key, ptrs, sizeof ptrs);
-    const int64_t cf[13] = {cfg.maxPaths, cfg.traceOversub, cfg.shadeOversub, cfg.walker, cfg.ldsStack,
+    const int64_t cf[12] = {cfg.maxPaths, cfg.traceOversub, cfg.shadeOversub, cfg.ldsStack,
                             cfg.shadeWaves, cfg.graphs, cfg.tailPaths, cfg.queueSort, cfg.ldsStackClosest,
                             (int64_t)nPaths, (int64_t)events, (int64_t)full};
     key = fnv(key, cf, sizeof cf);

@@ -124,3 +124,61 @@ def test_instanced_scene_bit_exact(orc, env):
     torch.cuda.synchronize()
     _, st = scene.closest(rays, stats=True)
     assert np.array_equal(cnt.cpu().numpy().astype(np.uint32), st)
+
+
+@pytest.fixture(scope="module")
+def queue_scene(orc, env):
+    """Instances in TLAS leaves of one and of several (coincident ones cannot
+    be split), meshes whose root is a leaf, both cullings; rays that start
+    inside and outside, short, with zero, infinite and NaN components."""
+    torch, accel, W = env
+    rng = np.random.default_rng(21)
+    one = (np.array([[-1, -1, 0], [1, -1, 0], [0, 1, 0]], np.float32), np.arange(3, dtype=np.uint32))
+    meshes = [W.sphere_mesh(20, 10), W.random_triangles(1500, mu=-2.0, seed=9), one]
+    mesh_idx, tr = [], []
+    for i in range(24):
+        q = rng.normal(size=4)
+        q /= np.linalg.norm(q)
+        t = W.trs(rng.random(3) * 5 - 2.5, q, float(rng.lognormal(0, 0.3)))
+        for _ in range(5 if i % 8 == 0 else 1):
+            mesh_idx.append(i % 3)
+            tr.append(t)
+    tr = np.array(tr)
+    mats = rng.integers(0, 2, len(mesh_idx))
+    scene = orc.assemble_scene([dict(positions=m[0], indices=m[1]) for m in meshes],
+                               dict(mesh=mesh_idx, transform=tr, material=mats), material_double_sided=[0, 1])
+    acc = accel.Accel([accel.Blas(m[0], m[1]) for m in meshes], mesh_idx, tr, material=mats,
+                      double_sided=[int(m) for m in mats])
+    n = 400_000
+    rays = np.zeros((n, 8), np.float32)
+    rays[:, 0:3] = rng.uniform(-4, 4, (n, 3))
+    rays[:, 4:7] = rng.normal(size=(n, 3))
+    rays[:, 3] = rng.uniform(0.0, 4.0, n)
+    bad = rng.integers(0, n, 4000)
+    rays[bad[:1500], rng.integers(4, 7, 1500)] = 0.0
+    rays[bad[1500:2000], 4:7] = 0.0
+    rays[bad[2000:3000], rng.integers(0, 7, 1000)] = np.nan
+    rays[bad[3000:], rng.integers(0, 7, 1000)] = np.inf
+    unbounded = rays.copy()  # closest-hit queries ignore tmax
+    unbounded[:, 3] = 9999.0
+    return scene, acc, rays, scene.closest(unbounded), scene.any(rays)
+
+
+# One ray, partial and full waves, one ray a wave on the whole grid and just
+# beyond, every lane used, chunks handed out dynamically.
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129, 2560, 5121, 40_000, 163_840, 163_841, 400_000])
+def test_query_sizes_bit_exact(orc, env, queue_scene, n):
+    torch, accel, W = env
+    scene, acc, rays, ref, occ = queue_scene
+    print(f"query of {n} rays", flush=True)
+    got = _gpu_closest(torch, acc, rays[:n])
+    _compare(scene, ref[:n], got, orc)
+    miss = got[:, 0] == 0
+    assert np.all(got[miss, 1:3] == 0xffffffff) and np.all(got[miss, 3].view(np.float32) == 9999.0)
+    assert np.all(got[miss, 4:8] == 0)
+    r = torch.from_numpy(rays[:n]).cuda()
+    o = torch.full((n + 1,), 7, dtype=torch.int32, device="cuda")
+    acc.trace_any(r, o)
+    torch.cuda.synchronize()
+    o = o.cpu().numpy()
+    assert np.array_equal(o[:n].astype(np.uint32), occ[:n]) and o[n] == 7
