@@ -322,6 +322,29 @@ def test_wavefront_equals_megakernel_large(env, orc):
     assert np.array_equal(out[0][0], out[1][0])
 
 
+# One pixel, a partial block, a block edge, rows that straddle blocks.
+@pytest.mark.parametrize("w,h", [(1, 1), (7, 5), (256, 1), (131, 4)])
+def test_read_pixels_kinds(env, w, h):
+    """Every pixel kind from the accumulators' sums in f64, rounded once."""
+    torch, render, scene = env
+    t = render.RenderTarget(render.RenderScene(scene.cornell_box()), w, h, bounces=3, max_samples=3)
+    t.render(3)
+    sums, counts = t.read_accumulators()
+    sums, n = sums[::-1], counts[::-1].astype(np.float64)[..., None]
+    total, hit = np.maximum(sums[..., 11:12], 1.0), sums[..., 7:8]
+    lum = (0.2126 * sums[..., 0:1] + 0.7152 * sums[..., 1:2] + 0.0722 * sums[..., 2:3]) / n
+    var = np.maximum(0.0, sums[..., 12:13] / n - lum * lum) / n
+    nrm = sums[..., 8:11]
+    valid = (nrm[..., 0:1] * nrm[..., 0:1] + nrm[..., 1:2] * nrm[..., 1:2] + nrm[..., 2:3] * nrm[..., 2:3]) > 0.1
+    zero, one = np.zeros_like(n), np.ones_like(n)
+    exp = dict(color=np.concatenate([sums[..., 0:3] / np.where(hit > 0, hit, total), sums[..., 3:4] / total], 2),
+               albedo=np.concatenate([sums[..., 4:7] / total, np.clip(hit / total, 0, 1)], 2),
+               normal=np.where(valid, np.concatenate([nrm / total * 0.5 + 0.5, one], 2), 0.0),
+               variance=np.concatenate([var, zero, zero, one], 2))
+    for kind, e in exp.items():
+        assert np.array_equal(t.read_pixels(kind), e.astype(np.float32)), kind
+
+
 @pytest.mark.parametrize("tuning", [
     dict(trace_kernel=0, lds_stack=16),
     dict(trace_kernel=1, lds_stack=16),
