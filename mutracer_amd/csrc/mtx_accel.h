@@ -174,6 +174,11 @@ using LaneStack = LaneStackT<kLdsStack>;
 // coverage test passes (intersectSceneQuery, intersect.wgsl.ts:643-646).
 constexpr uint32_t kSlotMasked = 2u;
 
+// Bits 2-4 of the same word: the shading class of the instance's material in
+// a render scene (which lobes its shading is likely to run). The shade kernel
+// groups hits by it; it changes no result.
+constexpr uint32_t kSlotClassShift = 2u, kSlotClassMask = 7u << kSlotClassShift;
+
 // Coverage test of any-hit queries that have no material data: every
 // triangle occludes.
 struct NoCoverage {

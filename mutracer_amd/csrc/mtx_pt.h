@@ -97,14 +97,18 @@ struct TargetObj;
 //   hitA closest hit t, barycentrics           hitB (instance slot or -1, triangle)
 //   qA/qB path-id queues of even/odd events
 //   s0..s3 shadow queue: (origin, tMax), (direction, path id), (payload, tri), slot
-//   counts[e] = length of event e's queue, counts[kWfShadowBase + e] = its shadow queue,
+//   counts[2e] = length of event e's queue, counts[2e + 3] = of its shadow queue (beside
+//                the length of queue e + 1: the shade kernel advances both with one atomic),
 //   counts[kWfXcdBase + x * kWfCtrStride + 2e (+1)] = next chunk handed out of XCD x's
 //                                           segment of event e's (shadow) queue
 //   counts[kWfTailFlag] = 1 + the event at which the tail kernel took over the
 //                         generation's remaining paths (0 while it has not)
 constexpr int kWfMaxEvents = 51;
-constexpr int kWfShadowBase = kWfMaxEvents + 1;
-constexpr int kWfXcdBase = (kWfShadowBase + kWfMaxEvents + 1 + 127) / 128 * 128;
+constexpr int wf_queue(int event) { return 2 * event; }
+constexpr int wf_shadow(int event) { return 2 * event + 3; }
+constexpr int kWfXcdBase = (wf_shadow(kWfMaxEvents) + 1 + 127) / 128 * 128;
+// Shading classes of hits (kSlotClassShift) and, last, paths without a hit.
+constexpr int kShadeMiss = 4, kShadeClasses = 5;
 constexpr int kWfXcds = 8;  // XCDs of an MI355X (counter segments per queue)
 constexpr int kWfCtrStride = 128;  // words of one XCD's counters, on lines of their own
 static_assert(2 * (kWfMaxEvents + 1) <= kWfCtrStride, "counters of one XCD");

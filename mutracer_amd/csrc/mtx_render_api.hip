@@ -423,6 +423,15 @@ static bool check_material_maps(const float *mat, uint32_t textureCount) {
   return textured;
 }
 
+// Shading class of a material (below kShadeMiss): hits of one class run mostly
+// the same lobes.
+static uint32_t shade_class(const float *m) {
+  if (m[MTX_MAT_TRANSMISSION_WEIGHT] > 0.0f || m[MTX_MAT_SUBSURFACE_WEIGHT] > 0.0f) return 3;
+  if (m[MTX_MAT_BASE_METALNESS] > 0.5f) return 2;
+  if (m[MTX_MAT_COAT_WEIGHT] > 0.0f || m[MTX_MAT_FUZZ_WEIGHT] > 0.0f) return 1;
+  return 0;
+}
+
 static std::shared_ptr<RenderSceneObj> create_scene(const mtx_scene_desc &D) {
   MTX_REQUIRE(D.struct_size >= offsetof(mtx_scene_desc, texture_count), MTX_INVALID_ARGUMENT,
               "mtx_scene_desc.struct_size too small");
@@ -469,8 +478,9 @@ static std::shared_ptr<RenderSceneObj> create_scene(const mtx_scene_desc &D) {
     MTX_REQUIRE(mat < D.material_count, MTX_INVALID_ARGUMENT, "instance material out of range");
     if (D.materials[(size_t)mat * MTX_MATERIAL_FLOATS + MTX_MAT_DOUBLE_SIDED] > 0.5f) d.double_sided = 1;
     // Shadow queries run the coverage test on instances of masked materials.
-    d.material_word = (d.material_word & ~kSlotMasked) |
-                      (D.materials[(size_t)mat * MTX_MATERIAL_FLOATS + MTX_MAT_ALPHA_MODE] == 1.0f ? kSlotMasked : 0u);
+    const float *m = D.materials + (size_t)mat * MTX_MATERIAL_FLOATS;
+    d.material_word = (d.material_word & ~(kSlotMasked | kSlotClassMask)) |
+                      (m[MTX_MAT_ALPHA_MODE] == 1.0f ? kSlotMasked : 0u) | (shade_class(m) << kSlotClassShift);
     R->triangles += D.meshes[d.blas_index].triangle_count;
   }
   R->accel = build_accel(R->blases, R->inst.data(), D.instance_count, tbins, D.flags, 0);

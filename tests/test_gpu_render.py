@@ -322,6 +322,25 @@ def test_wavefront_equals_megakernel_large(env, orc):
     assert np.array_equal(out[0][0], out[1][0])
 
 
+# A wave of the shade kernel takes 64 paths at a time from 2048 waves' shares
+# of the queue: a partial wave, one share each, two (a class fills once), five
+# (classes fill repeatedly, two at once, leftovers of several).
+@pytest.mark.parametrize("w,h,spp", [(9, 5, 1), (256, 128, 4), (320, 200, 4), (400, 250, 6)])
+@pytest.mark.parametrize("tail_paths", [0, 1 << 16])
+def test_shading_classes_match_oracle(env, orc, w, h, spp, tail_paths):
+    """Paths shaded grouped by what they hit (diffuse, coat, metal, glass,
+    nothing) give the oracle's sums, with and without the tail kernel."""
+    torch, render, scene = env
+    sc = scene.instanced_field(n_instances=13, freq=5, env_size=(64, 32))
+    t = render.RenderTarget(render.RenderScene(sc), w, h, bounces=3, direct_light_candidates=2, max_samples=spp)
+    t.set_tuning(tail_paths=tail_paths)
+    t.render(spp)
+    sums, counts = t.read_accumulators()
+    ref = orc.OracleRenderer(sc, w, h, bounces=3, candidates=2, max_samples=spp).render(0, spp)
+    assert np.all(counts == spp)
+    assert np.array_equal(sums, ref)
+
+
 # One pixel, a partial block, a block edge, rows that straddle blocks.
 @pytest.mark.parametrize("w,h", [(1, 1), (7, 5), (256, 1), (131, 4)])
 def test_read_pixels_kinds(env, w, h):
