@@ -66,7 +66,7 @@ k_trace(const AccelView *__restrict__ viewp, const mtx_ray *__restrict__ rays, u
     if (!any) hits[i] = mtx_hit{0u, -1, -1, kRayMaxDistance, {0.0f, 0.0f, 0.0f}, 0u};
     if (kMode == 3) hits[i].visits = c.boxes + c.tris;
   };
-  trace_queue<kMode == 1, (kMode >= 2), false, false>(
+  trace_queue<kMode == 1, (kMode >= 2), false, false, false>(
       n, ctr, acc, doubleSided, st, load, hit, covers, done);
 }
 

@@ -57,7 +57,9 @@ struct WorkQueue {
     return true;
   }
 
-  __device__ __forceinline__ WorkQueue(uint32_t n_, uint32_t *ctr_) : n(n_), ctr(ctr_) {
+  // `reverse`: first chunks go to the waves from the grid's end, for the
+  // second of two queues that one launch empties.
+  __device__ __forceinline__ WorkQueue(uint32_t n_, uint32_t *ctr_, bool reverse) : n(n_), ctr(ctr_) {
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
     const uint32_t per = (uint32_t)(((uint64_t)n + waves - 1u) / waves);
     lanes = (int)min(64u, max(1u, per));
@@ -67,7 +69,8 @@ struct WorkQueue {
     refillMin = min(lanes, kRefill);
     seg = blockIdx.x % (uint32_t)kXcds;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t c = seg_lo(seg) + (blockIdx.x / (uint32_t)kXcds) * (blockDim.x >> 6) + wave;
+    const uint32_t rank = (blockIdx.x / (uint32_t)kXcds) * (blockDim.x >> 6) + wave;
+    const uint32_t c = seg_lo(seg) + (reverse ? seg_waves(seg) - 1u - rank : rank);
     base = limit = 0;
     open = true;
     if (c < seg_lo(seg + 1u)) set(c);

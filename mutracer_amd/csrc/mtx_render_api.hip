@@ -521,12 +521,15 @@ static std::shared_ptr<RenderSceneObj> create_scene(const mtx_scene_desc &D) {
   v.envGuide = hasEnv ? R->envGuide.ptr : nullptr;
   v.emissive = E.weight.empty() ? nullptr : R->emissive.ptr;
   v.emissiveCount = (uint32_t)E.weight.size();
-  v.features = 0;
+  v.features = textured ? 0u : kSceneOpaque;
   for (uint32_t m = 0; m < D.material_count; m++) {
     const float *mat = D.materials + (size_t)m * MTX_MATERIAL_FLOATS;
     if (mat[MTX_MAT_FUZZ_WEIGHT] > 0.0f || mat[MTX_MAT_SUBSURFACE_WEIGHT] > 0.0f || mat[MTX_MAT_THIN_WALLED] > 0.5f)
       v.features |= kSceneFull;
     if (mat[MTX_MAT_ALPHA_MODE] == 1.0f) v.features |= kSceneMasked;
+    if (!(mat[MTX_MAT_ALPHA_MODE] == 0.0f && mat[MTX_MAT_TRANSMISSION_WEIGHT] < 0.001f &&
+          mat[MTX_MAT_SUBSURFACE_WEIGHT] < 0.001f))
+      v.features &= ~kSceneOpaque;
   }
   if (textured) {
     v.features |= kSceneFull | kSceneTextured;
@@ -667,6 +670,7 @@ std::shared_ptr<TargetObj> create_target(std::shared_ptr<RenderSceneObj> scene, 
   T->params = params_from(s, cam);
   T->kernel = s.kernel;
   if (s.max_paths_in_flight) T->wfConfig.maxPaths = s.max_paths_in_flight;
+  T->wfConfig.tailPaths = default_tail_paths(scene->triangles);
   const size_t N = (size_t)s.width * s.height;
   T->planes.alloc(N * 13);
   T->count.alloc(N);
@@ -1253,6 +1257,7 @@ static uint32_t server_round(ServerObj &S, hipStream_t s, bool &idle) {
   std::vector<std::pair<std::shared_ptr<ServerJob>, uint32_t>> parts;
   uint32_t paths = 0, pixels = 0;
   int eventLimit = 0;
+  uint64_t triangles = 0;  // of the round's largest scene
   for (uint64_t h : S.running) {
     if (slots.size() >= S.maxJobs) break;
     auto J = S.jobs.at(h);
@@ -1276,7 +1281,8 @@ static uint32_t server_round(ServerObj &S, hipStream_t s, bool &idle) {
     parts.emplace_back(J, g);
     paths += g * J->params.pixelCount;
     pixels += J->params.pixelCount;
-    eventLimit = std::max(eventLimit, std::min((int)J->params.bounces * 3, 50));
+    eventLimit = std::max(eventLimit, event_limit(js.scene, js.params));
+    triangles = std::max(triangles, J->scene->triangles);
     if (J->state == MTX_JOB_QUEUED) { J->state = MTX_JOB_RUNNING; J->startMs = now_ms(); }
   }
   idle = slots.empty();
@@ -1298,6 +1304,7 @@ static uint32_t server_round(ServerObj &S, hipStream_t s, bool &idle) {
       if (!S.graph.own) MTX_HIP(hipStreamCreate(&S.graph.own));
       rs = S.graph.own;
     }
+    S.cfg.tailPaths = default_tail_paths(triangles);
     S.slots.upload(slots.data(), slots.size(), rs);
     launch_generation_multi(S.slots.ptr, (uint32_t)slots.size(), paths, pixels, eventLimit, S.rays.ptr, S.wf, S.cfg,
                             rs, full, masked, nullptr, &S.graph);

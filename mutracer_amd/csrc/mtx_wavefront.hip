@@ -147,52 +147,6 @@ __device__ __forceinline__ void flush_work(uint64_t *work, const uint64_t (&v0)[
   }
 }
 
-template <bool kMulti, bool kCount, int kLds>
-__global__ void __launch_bounds__(kWfTraceBlock, kTraceWaves)
-k_wf_trace(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spill) {
-  __shared__ int32_t lds[kLds * kWfTraceBlock];
-  const uint32_t n = W.counts[wf_queue(event)];
-  if (n == 0u || W.counts[kWfTailFlag]) return;
-  LaneStackT<kLds> st{lds + threadIdx.x, kWfTraceBlock,
-                      spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
-  const uint32_t *q = queue_of(W, event);
-  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
-  AccelView one{};
-  if (!kMulti) one = *L.one.scene.accel;
-  uint64_t boxes = 0, tris = 0, instances = 0, hits = 0;
-  auto load = [&](uint32_t i, RayIn &r) {
-    const uint32_t p = q[i];
-    r.o = f3of(W.o[p]);
-    r.d = f3of(W.d[p]);
-    r.tMax = kRayMaxDistance;
-    r.curTri = fint(W.beta[p].w);
-    r.curSlot = fint(W.alb[p].w);
-    if (kMulti) r.acc = job_of<true>(L, W, p).scene.accel;
-    r.id = p;
-  };
-  auto hit = [&](uint32_t p, float t, f3 b, int32_t slot, int32_t tri, int32_t) {
-    W.hitA[p] = make_float4(t, b.x, b.y, b.z);
-    W.hitB[p] = make_int2(slot, tri);
-  };
-  auto covers = [](uint32_t, int32_t, int32_t, f3) { return true; };
-  auto done = [&](uint32_t p, bool any, const TraceCounters &c) {
-    if (!any) W.hitB[p] = make_int2(-1, -1);
-    if (kCount) {
-      boxes += c.boxes;
-      tris += c.tris;
-      instances += c.instances;
-      hits += any ? 1u : 0u;
-    }
-  };
-  trace_queue<false, kCount, kMulti, false>(n, W.counts + kWfXcdBase + 2 * event, one, event != 0, st, load, hit,
-                                            covers, done);
-  if (kCount) {
-    const uint64_t v[5] = {(blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u, boxes, tris, instances, hits};
-    const int slots[5] = {kWorkClosestRays, kWorkBoxes, kWorkTris, kWorkInstances, kWorkHits};
-    flush_work(L.work, v, slots);
-  }
-}
-
 // Reserves a slot in queue `event` + 1 per lane with `next` and one in event's
 // shadow queue per lane with `shadow`, in one atomic; all lanes of the wave.
 __device__ __forceinline__ void wave_append2(uint32_t *counts, int event, bool next, bool shadow, uint32_t &slot,
@@ -223,7 +177,7 @@ __device__ __forceinline__ void wave_append2(uint32_t *counts, int event, bool n
 // of an instruction are active and shading takes 48.6 ms instead of 64.4; the
 // loads' latency at two waves per SIMD bounds it now (the VALU issues 41% of
 // the cycles; three waves spill: 72 ms). Both queues advance with one atomic
-// per wave. Chunks of fewer than 64 paths for short queues measured the same.
+// per wave.
 template <bool kMulti, int kWaves, bool kFull>
 __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaunch L, WfBuffers W, int event) {
   __shared__ uint32_t binMem[kWfShadeBlock / 64][kShadeClasses][128];
@@ -239,7 +193,11 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
   uint32_t cnt[kShadeClasses];
 #pragma unroll
   for (int c = 0; c < kShadeClasses; c++) cnt[c] = 0u;
-  uint32_t at = wave * 64u;
+  // A queue shorter than the grid's lanes is spread over the waves, as in
+  // WorkQueue: fewer paths to diverge within a wave (late events 2-6% of a
+  // frame with deep scenes; nothing for queues that fill the grid).
+  const uint32_t per = min(64u, max(1u, (n + nWaves - 1u) / nWaves));
+  uint32_t at = wave * per;
   while (true) {
     // Take paths until a class has a wave's worth (two can get it at once).
     bool full = false;
@@ -247,7 +205,7 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
     for (int c = 0; c < kShadeClasses; c++) full = full || cnt[c] >= 64u;
     while (!full && at < n) {
       const uint32_t i = at + lane;
-      const bool have = i < n;
+      const bool have = lane < per && i < n;
       uint32_t p = 0;
       int cls = -1;
       if (have) {
@@ -264,7 +222,7 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
         cnt[c] += (uint32_t)__popcll(m);
         full = full || cnt[c] >= 64u;
       }
-      at = n - at > nWaves * 64u ? at + nWaves * 64u : n;
+      at = n - at > nWaves * per ? at + nWaves * per : n;
     }
     __builtin_amdgcn_wave_barrier();
     // The last 64 paths of a full class, or what the classes have left.
@@ -371,17 +329,52 @@ __device__ __forceinline__ void add_payload(const WfBuffers &W, uint32_t p, floa
   W.li[p] = l;
 }
 
-template <bool kMulti, bool kCount, int kLds, bool kAlpha>
-__global__ void __launch_bounds__(kWfTraceBlock, kTraceWaves)
-k_wf_shadow(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spill) {
-  __shared__ int32_t lds[kLds * kWfTraceBlock];
-  const uint32_t n = W.counts[wf_shadow(event)];
-  if (n == 0u || W.counts[kWfTailFlag]) return;
-  LaneStackT<kLds> st{lds + threadIdx.x, kWfTraceBlock,
-                      spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
+// Closest hits of event's queue (n paths).
+template <bool kMulti, bool kCount, class Stack>
+__device__ __forceinline__ void closest_hits(const WfLaunch &L, const WfBuffers &W, int event, uint32_t n,
+                                             const AccelView &one, Stack &st) {
+  const uint32_t *q = queue_of(W, event);
   if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
-  AccelView one{};
-  if (!kMulti) one = *L.one.scene.accel;
+  uint64_t boxes = 0, tris = 0, instances = 0, hits = 0;
+  auto load = [&](uint32_t i, RayIn &r) {
+    const uint32_t p = q[i];
+    r.o = f3of(W.o[p]);
+    r.d = f3of(W.d[p]);
+    r.tMax = kRayMaxDistance;
+    r.curTri = fint(W.beta[p].w);
+    r.curSlot = fint(W.alb[p].w);
+    if (kMulti) r.acc = job_of<true>(L, W, p).scene.accel;
+    r.id = p;
+  };
+  auto hit = [&](uint32_t p, float t, f3 b, int32_t slot, int32_t tri, int32_t) {
+    W.hitA[p] = make_float4(t, b.x, b.y, b.z);
+    W.hitB[p] = make_int2(slot, tri);
+  };
+  auto covers = [](uint32_t, int32_t, int32_t, f3) { return true; };
+  auto done = [&](uint32_t p, bool any, const TraceCounters &c) {
+    if (!any) W.hitB[p] = make_int2(-1, -1);
+    if (kCount) {
+      boxes += c.boxes;
+      tris += c.tris;
+      instances += c.instances;
+      hits += any ? 1u : 0u;
+    }
+  };
+  trace_queue<false, kCount, kMulti, false, false>(n, W.counts + kWfXcdBase + 2 * event, one, event != 0, st, load,
+                                                   hit, covers, done);
+  if (kCount) {
+    const uint64_t v[5] = {(blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u, boxes, tris, instances, hits};
+    const int slots[5] = {kWorkClosestRays, kWorkBoxes, kWorkTris, kWorkInstances, kWorkHits};
+    flush_work(L.work, v, slots);
+  }
+}
+
+// Any hit for event's shadow queue (n rays); adds the payload of each
+// unoccluded ray to its path's radiance.
+template <bool kMulti, bool kCount, bool kAlpha, class Stack>
+__device__ __forceinline__ void shadow_rays(const WfLaunch &L, const WfBuffers &W, int event, uint32_t n,
+                                            const AccelView &one, Stack &st) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd((unsigned long long *)L.rays, (unsigned long long)n);
   uint64_t boxes = 0, tris = 0, instances = 0;
   auto path = [&](uint32_t i) { return (uint32_t)fint(W.s1[i].w); };
   auto load = [&](uint32_t i, RayIn &r) {
@@ -410,13 +403,34 @@ k_wf_shadow(const WfLaunch L, WfBuffers W, int event, int32_t *__restrict__ spil
       instances += c.instances;
     }
   };
-  trace_queue<true, kCount, kMulti, kAlpha>(n, W.counts + kWfXcdBase + 2 * event + 1, one, true, st, load, hit, covers,
-                                            done);
+  trace_queue<true, kCount, kMulti, kAlpha, true>(n, W.counts + kWfXcdBase + 2 * event + 1, one, true, st, load, hit,
+                                                  covers, done);
   if (kCount) {
     const uint64_t v[4] = {boxes, tris, instances, (blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u};
     const int slots[4] = {kWorkShadowBoxes, kWorkShadowTris, kWorkShadowInstances, kWorkShadowRays};
     flush_work(L.work, v, slots);
   }
+}
+
+// The ray queries between two shade kernels: closest hits of event's queue
+// and the shadow rays of the event before (either may be left out: a negative
+// event). They are independent (a shadow ray adds to its path's radiance,
+// which no closest-hit query reads), so one launch runs both and its end is
+// the later of the two instead of their sum: a late event with a few thousand
+// rays of each kind takes one latency chain.
+template <bool kMulti, bool kCount, int kLds, bool kAlpha>
+__global__ void __launch_bounds__(kWfTraceBlock, kTraceWaves)
+k_wf_query(const WfLaunch L, WfBuffers W, int event, int shadowEvent, int32_t *__restrict__ spill) {
+  __shared__ int32_t lds[kLds * kWfTraceBlock];
+  const uint32_t n = event >= 0 ? W.counts[wf_queue(event)] : 0u;
+  const uint32_t m = shadowEvent >= 0 ? W.counts[wf_shadow(shadowEvent)] : 0u;
+  if ((n | m) == 0u || W.counts[kWfTailFlag]) return;
+  LaneStackT<kLds> st{lds + threadIdx.x, kWfTraceBlock,
+                      spill + ((size_t)blockIdx.x * kWfTraceBlock + threadIdx.x) * (kMaxStack - kLds)};
+  AccelView one{};
+  if (!kMulti) one = *L.one.scene.accel;
+  if (n) closest_hits<kMulti, kCount>(L, W, event, n, one, st);
+  if (m) shadow_rays<kMulti, kCount, kAlpha>(L, W, shadowEvent, m, one, st);
 }
 
 // Tail of a generation: once event `event`'s queue holds at most `tailPaths`
@@ -645,61 +659,46 @@ WfBuffers WfBuffers::Owner::view(uint32_t nPaths, bool sort) const {
   return W;
 }
 
-template <bool kMulti, bool kShadow, int kLds>
-static void launch_trace_lds(uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W, int e,
+template <bool kMulti, int kLds>
+static void launch_query_lds(uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W, int e, int se,
                              int32_t *spill) {
-  if (kShadow) {
-    if (L.masked) {
-      if (L.work)
-        hipLaunchKernelGGL((k_wf_shadow<kMulti, true, kLds, true>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                           spill);
-      else
-        hipLaunchKernelGGL((k_wf_shadow<kMulti, false, kLds, true>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                           spill);
-    } else if (L.work) {
-      hipLaunchKernelGGL((k_wf_shadow<kMulti, true, kLds, false>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                         spill);
-    } else {
-      hipLaunchKernelGGL((k_wf_shadow<kMulti, false, kLds, false>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e,
-                         spill);
-    }
+  const dim3 g(grid), b(kWfTraceBlock);
+  if (L.masked) {
+    if (L.work) hipLaunchKernelGGL((k_wf_query<kMulti, true, kLds, true>), g, b, 0, s, L, W, e, se, spill);
+    else hipLaunchKernelGGL((k_wf_query<kMulti, false, kLds, true>), g, b, 0, s, L, W, e, se, spill);
   } else {
-    if (L.work)
-      hipLaunchKernelGGL((k_wf_trace<kMulti, true, kLds>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e, spill);
-    else
-      hipLaunchKernelGGL((k_wf_trace<kMulti, false, kLds>), dim3(grid), dim3(kWfTraceBlock), 0, s, L, W, e, spill);
+    if (L.work) hipLaunchKernelGGL((k_wf_query<kMulti, true, kLds, false>), g, b, 0, s, L, W, e, se, spill);
+    else hipLaunchKernelGGL((k_wf_query<kMulti, false, kLds, false>), g, b, 0, s, L, W, e, se, spill);
   }
 }
-// Closest-hit (kShadow false) or any-hit launch with the configured LDS stack depth.
-template <bool kMulti, bool kShadow>
-static void launch_trace(const WfConfig &cfg, uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W,
-                         int e, int32_t *spill) {
-  const int depth = (!kShadow && cfg.ldsStackClosest) ? cfg.ldsStackClosest : cfg.ldsStack;
-  if (depth <= 16) launch_trace_lds<kMulti, kShadow, 16>(grid, s, L, W, e, spill);
-  else if (depth <= 24) launch_trace_lds<kMulti, kShadow, 24>(grid, s, L, W, e, spill);
-  else launch_trace_lds<kMulti, kShadow, 32>(grid, s, L, W, e, spill);
+// LDS stack entries of the query kernel: the larger of the two settings.
+static int query_lds(const WfConfig &cfg) {
+  const int d = std::max(cfg.ldsStack, cfg.ldsStackClosest);
+  return d <= 16 ? 16 : (d <= 24 ? 24 : 32);
+}
+template <bool kMulti>
+static void launch_query(const WfConfig &cfg, uint32_t grid, hipStream_t s, const WfLaunch &L, const WfBuffers &W,
+                         int e, int se, int32_t *spill) {
+  switch (query_lds(cfg)) {
+    case 16: launch_query_lds<kMulti, 16>(grid, s, L, W, e, se, spill); break;
+    case 24: launch_query_lds<kMulti, 24>(grid, s, L, W, e, se, spill); break;
+    default: launch_query_lds<kMulti, 32>(grid, s, L, W, e, se, spill); break;
+  }
 }
 
 struct Grids {
-  uint32_t trace, shadow, shade, tail, cus;
+  uint32_t query, shade, tail, cus;
 };
 static Grids grids_for(const WfConfig &cfg) {
-  static int closestBpc[3] = {0, 0, 0}, shadowBpc[3] = {0, 0, 0}, shadeBpc[5] = {0, 0, 0, 0, 0}, tailBpc = 0;
+  static int queryBpc[3] = {0, 0, 0}, shadeBpc[5] = {0, 0, 0, 0, 0}, tailBpc = 0;
   const int cus = cu_count();
-  auto level = [](int d) { return d <= 16 ? 0 : (d <= 24 ? 1 : 2); };
-  const int li = level(cfg.ldsStack), lc = level(cfg.ldsStackClosest ? cfg.ldsStackClosest : cfg.ldsStack);
-  if (!closestBpc[lc]) {
-    const void *t = lc == 0 ? (const void *)k_wf_trace<false, false, 16>
-                  : lc == 1 ? (const void *)k_wf_trace<false, false, 24> : (const void *)k_wf_trace<false, false, 32>;
-    closestBpc[lc] = blocks_per_cu(t, kWfTraceBlock, 0);
+  const int lds = query_lds(cfg), lq = lds / 8 - 2;
+  if (!queryBpc[lq]) {
+    const void *k = lds == 16   ? (const void *)k_wf_query<false, false, 16, false>
+                    : lds == 24 ? (const void *)k_wf_query<false, false, 24, false>
+                                : (const void *)k_wf_query<false, false, 32, false>;
+    queryBpc[lq] = blocks_per_cu(k, kWfTraceBlock, 0);
   }
-  if (!shadowBpc[li]) {
-    const void *a = li == 0   ? (const void *)k_wf_shadow<false, false, 16, false>
-                    : li == 1 ? (const void *)k_wf_shadow<false, false, 24, false>
-                              : (const void *)k_wf_shadow<false, false, 32, false>;
-    shadowBpc[li] = blocks_per_cu(a, kWfTraceBlock, 0);
-  }
-
   const int sw = std::min(4, std::max(1, cfg.shadeWaves));
   if (!shadeBpc[sw]) {
     const void *k = sw == 1 ? (const void *)k_wf_shade<false, 1, true> : sw == 2 ? (const void *)k_wf_shade<false, 2, true>
@@ -710,8 +709,7 @@ static Grids grids_for(const WfConfig &cfg) {
   Grids g;
   g.cus = (uint32_t)cus;
   g.tail = (uint32_t)(cus * tailBpc);
-  g.trace = (uint32_t)(cus * closestBpc[lc] * std::max(1, cfg.traceOversub));
-  g.shadow = (uint32_t)(cus * shadowBpc[li] * std::max(1, cfg.traceOversub));
+  g.query = (uint32_t)(cus * queryBpc[lq] * std::max(1, cfg.traceOversub));
   g.shade = (uint32_t)(cus * shadeBpc[sw] * std::max(1, cfg.shadeOversub));
   return g;
 }
@@ -759,6 +757,12 @@ static void run_generation(const WfLaunch &L, const WfBuffers &W, int eventLimit
   hipLaunchKernelGGL(k_wf_reset, dim3(1), dim3(256), 0, s, W, select ? 0u : W.nPaths);
   hipLaunchKernelGGL(k_wf_generate<kMulti>, dim3(genGrid), dim3(256), 0, s, L, W, select ? 1 : 0);
   te();
+  // Per event: closest hits, shading, shadow rays. The shadow rays of an
+  // event share a launch with the next event's closest hits, except where the
+  // tail kernel may take over in between (it continues the paths' radiance)
+  // and where the launches are timed by class. The last event shades without
+  // sampling, so it has no shadow rays.
+  const bool fused = !cfg.tailPaths && !timer;
   for (int e = 0; e <= eventLimit; e++) {
     if (cfg.tailPaths) {
       tb(5);
@@ -767,16 +771,18 @@ static void run_generation(const WfLaunch &L, const WfBuffers &W, int eventLimit
       te();
     }
     tb(1);
-    launch_trace<kMulti, false>(cfg, g.trace, s, L, W, e, spill);
+    launch_query<kMulti>(cfg, g.query, s, L, W, e, fused ? e - 1 : -1, spill);
     te();
     tb(2);
     if (full) launch_shade<kMulti, true>(cfg, g, s, L, W, e);
     else launch_shade<kMulti, false>(cfg, g, s, L, W, e);
     if (W.qSort && e < eventLimit) hipLaunchKernelGGL(k_wf_gather, dim3(genGrid), dim3(256), 0, s, W, e + 1);
     te();
-    tb(3);
-    launch_trace<kMulti, true>(cfg, g.shadow, s, L, W, e, spill);
-    te();
+    if (!fused && e < eventLimit) {
+      tb(3);
+      launch_query<kMulti>(cfg, g.query, s, L, W, -1, e, spill);
+      te();
+    }
   }
   const uint32_t accGrid = std::min<uint32_t>((pixels + 255) / 256, g.cus * 16u);
   tb(0);
@@ -823,8 +829,8 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
   const uint32_t maxPaths = std::max<uint32_t>(cfg.maxPaths, p0.pixelCount);
   const uint32_t genMax = std::max<uint32_t>(1u, maxPaths / p0.pixelCount);
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(std::max(g.trace, g.shadow), g.tail), kWfTraceBlock);
-  const int eventLimit = std::min((int)p0.bounces * 3, 50);
+  int32_t *spill = spill_for(s, std::max(g.query, g.tail), kWfTraceBlock);
+  const int eventLimit = event_limit(scene, p0);
   uint32_t done = 0;
   while (done < p0.samples) {
     const uint32_t gen = std::min(genMax, p0.samples - done);
@@ -895,7 +901,7 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
   if (!nJobs || !nPaths) return;
   MTX_REQUIRE(nJobs <= kMaxJobsPerRound, MTX_INVALID_ARGUMENT, "too many jobs in one round");
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(std::max(g.trace, g.shadow), g.tail), kWfTraceBlock);
+  int32_t *spill = spill_for(s, std::max(g.query, g.tail), kWfTraceBlock);
   buf.ensure(nPaths, cfg.queueSort);
   const WfBuffers W = buf.view(nPaths, cfg.queueSort);
   WfLaunch L;

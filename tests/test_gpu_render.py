@@ -329,7 +329,8 @@ def test_wavefront_equals_megakernel_large(env, orc):
 @pytest.mark.parametrize("tail_paths", [0, 1 << 16])
 def test_shading_classes_match_oracle(env, orc, w, h, spp, tail_paths):
     """Paths shaded grouped by what they hit (diffuse, coat, metal, glass,
-    nothing) give the oracle's sums, with and without the tail kernel."""
+    nothing) give the oracle's sums, with the shadow rays of an event in the
+    next event's launch (no tail) and in their own."""
     torch, render, scene = env
     sc = scene.instanced_field(n_instances=13, freq=5, env_size=(64, 32))
     t = render.RenderTarget(render.RenderScene(sc), w, h, bounces=3, direct_light_candidates=2, max_samples=spp)
@@ -339,6 +340,24 @@ def test_shading_classes_match_oracle(env, orc, w, h, spp, tail_paths):
     ref = orc.OracleRenderer(sc, w, h, bounces=3, candidates=2, max_samples=spp).render(0, spp)
     assert np.all(counts == spp)
     assert np.array_equal(sums, ref)
+
+
+@pytest.mark.parametrize("kind", ["diffuse", "glass", "masked", "subsurface"])
+@pytest.mark.parametrize("bounces", [0, 1, 2, 7])
+def test_event_limit_of_opaque_scenes(env, orc, kind, bounces):
+    """Scenes that let no path past `bounces` + 1 events launch no more of
+    them; one transmitting, masked or subsurface material lifts that."""
+    torch, render, scene = env
+    sc = scene.cornell_box()
+    more = dict(diffuse={}, glass=dict(transmission_weight=1.0, specular_roughness=0.1),
+                masked=dict(alpha_mode="mask", opacity=0.2, alpha_cutoff=0.5),
+                subsurface=dict(subsurface_weight=0.6))[kind]
+    sc.materials.append(scene.Material(base_color=(0.7, 0.8, 0.9), **more))
+    sc.instance_material[-1] = len(sc.materials) - 1
+    t = render.RenderTarget(render.RenderScene(sc), 40, 32, bounces=bounces, max_samples=4)
+    t.render(4)
+    sums, _ = t.read_accumulators()
+    assert np.array_equal(sums, orc.OracleRenderer(sc, 40, 32, bounces=bounces, candidates=1, max_samples=4).render(0, 4))
 
 
 # One pixel, a partial block, a block edge, rows that straddle blocks.
