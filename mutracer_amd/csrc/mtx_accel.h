@@ -24,6 +24,43 @@
 
 namespace mtx {
 
+// Traversal reads nodes, triangles and instance slots through global
+// address-space pointers: loads through generic (flat) pointers also count
+// against the LDS counter, so every wait for a node would wait for the LDS
+// stack's operations too.
+#if defined(__HIP_DEVICE_COMPILE__)
+#define MTX_AS_GLOBAL __attribute__((address_space(1)))
+#define MTX_AS_LDS __attribute__((address_space(3)))
+#else
+#define MTX_AS_GLOBAL
+#define MTX_AS_LDS
+#endif
+template <class T>
+__device__ __forceinline__ const MTX_AS_GLOBAL T *as_global(const T *p) {
+  return (const MTX_AS_GLOBAL T *)p;
+}
+// The same for code that goes on with a generic pointer: the compiler infers
+// the address space from the cast.
+template <class T>
+MTX_HD T *global_ptr(T *p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (T *)(MTX_AS_GLOBAL T *)p;
+#else
+  return p;
+#endif
+}
+// A pointer kept in device memory: its target is read through the global
+// address space (a pointer loaded from memory is generic to the compiler, and
+// its loads would be flat).
+template <class T>
+struct GlobalPtr {
+  T *p;
+  GlobalPtr() = default;
+  MTX_HD GlobalPtr(T *q) : p(q) {}
+  MTX_HD operator T *() const { return global_ptr(p); }
+  MTX_HD T *operator->() const { return global_ptr(p); }
+};
+
 struct TNode {
   float4 a, b, c, d;
 };
@@ -44,23 +81,6 @@ struct InstSlot {
 static_assert(sizeof(TNode) == 64, "TNode");
 static_assert(sizeof(TriRec) == 48, "TriRec");
 static_assert(sizeof(InstSlot) == 128, "InstSlot");
-
-// Traversal reads nodes, triangles and instance slots through global
-// address-space pointers: loads through generic (flat) pointers also count
-// against the LDS counter, so every wait for a node would wait for the LDS
-// stack's operations too.
-#if defined(__HIP_DEVICE_COMPILE__)
-#define MTX_AS_GLOBAL __attribute__((address_space(1)))
-#define MTX_AS_LDS __attribute__((address_space(3)))
-#else
-#define MTX_AS_GLOBAL
-#define MTX_AS_LDS
-#endif
-template <class T>
-__device__ __forceinline__ const MTX_AS_GLOBAL T *as_global(const T *p) {
-  return (const MTX_AS_GLOBAL T *)p;
-}
-
 
 struct AccelView {
   const TNode *tlasNodes;

@@ -10,11 +10,11 @@ namespace mtx {
 // Shading data per instance slot (leaf order, parallel to InstSlot).
 struct ShadeSlot {
   float4 l2w0, l2w1, l2w2, l2w3;  // local-to-world columns (xyz)
-  const float *normals;           // source mesh vertex normals (xyz)
-  const uint32_t *indices;        // source mesh triangle indices
+  GlobalPtr<const float> normals;           // source mesh vertex normals (xyz)
+  GlobalPtr<const uint32_t> indices;        // source mesh triangle indices
   uint32_t material;
   float color[3];
-  const float *uvs, *uvs1;        // source mesh UV0 / UV1 (xy), or null
+  GlobalPtr<const float> uvs, uvs1;        // source mesh UV0 / UV1 (xy), or null
 };
 static_assert(sizeof(ShadeSlot) == 112, "ShadeSlot");
 
@@ -36,28 +36,28 @@ struct LightChoice {
 // Packed OpenPBR material (32 floats) and rect light (16 floats); the field
 // offsets are documented with mtx_material_desc / mtx_light_desc in mtx.h.
 struct GpuScene {
-  const AccelView *accel;
-  const ShadeSlot *shade;
-  const float *materials;
-  const float *lights;
-  const float *lightPmf;       // per light selection pmf
-  const LightChoice *choices;
+  GlobalPtr<const AccelView> accel;
+  GlobalPtr<const ShadeSlot> shade;
+  GlobalPtr<const float> materials;
+  GlobalPtr<const float> lights;
+  GlobalPtr<const float> lightPmf;       // per light selection pmf
+  GlobalPtr<const LightChoice> choices;
   int32_t choiceCount;
   uint32_t lightCount;
   float envPmf;
   float lightWeightTotal;
-  const float4 *env;           // RGBA f32, envH rows of envW
-  const float2 *envCdf;        // (envW + 2) x (envH + 1)
+  GlobalPtr<const float4> env;           // RGBA f32, envH rows of envW
+  GlobalPtr<const float2> envCdf;        // (envW + 2) x (envH + 1)
   uint32_t envW, envH;
-  const float *lut;            // 32 x 2177 energy tables
-  const float4 *emissive;      // 3 per emissive triangle: (p0, pmf), (p1, area), (p2, material), world space
+  GlobalPtr<const float> lut;            // 32 x 2177 energy tables
+  GlobalPtr<const float4> emissive;      // 3 per emissive triangle: (p0, pmf), (p1, area), (p2, material), world space
   uint32_t emissiveCount;
   uint32_t features;           // kSceneFull when a material has fuzz, subsurface, a thin wall or a texture
-  const uint16_t *envGuide;    // search brackets of envCdf (kEnvGuideRows + 1, then envH x (kEnvGuideCols + 1)), or null
-  const GpuTexture *textures;  // material textures, or null (no material has a map)
-  const uint32_t *texels8;     // RGBA8 texel pool
-  const float4 *texels32;      // RGBA32F texel pool
-  const float4 *emissiveUv;    // 3 per emissive triangle: (uv0, uv1), (uv2, uv1_0), (uv1_1, uv1_2), with textures
+  GlobalPtr<const uint16_t> envGuide;    // search brackets of envCdf (kEnvGuideRows + 1, then envH x (kEnvGuideCols + 1)), or null
+  GlobalPtr<const GpuTexture> textures;  // material textures, or null (no material has a map)
+  GlobalPtr<const uint32_t> texels8;     // RGBA8 texel pool
+  GlobalPtr<const float4> texels32;      // RGBA32F texel pool
+  GlobalPtr<const float4> emissiveUv;    // 3 per emissive triangle: (uv0, uv1), (uv2, uv1_0), (uv1_1, uv1_2), with textures
 };
 // Bins of the environment CDF guide tables: bin k of the marginal (of row
 // y's conditional) CDF holds the index its search returns for the sample
@@ -82,12 +82,12 @@ struct RenderParams {
 
 // FP64 accumulators, one plane per channel (13 planes) + u32 sample counts.
 struct Accumulators {
-  double *planes;  // 13 * pixels
-  uint32_t *count;
+  GlobalPtr<double> planes;  // 13 * pixels
+  GlobalPtr<uint32_t> count;
   uint64_t *rays;  // traced rays (camera + continuation + shadow)
   uint32_t pixels;
   uint64_t *work;  // optional: box tests, triangle tests, instance visits, hits, shadow rays
-  const float *targets = nullptr;  // optional per-pixel sample targets (adaptive sampling)
+  GlobalPtr<const float> targets = nullptr;  // optional per-pixel sample targets (adaptive sampling)
 };
 
 struct RenderSceneObj;

@@ -82,7 +82,7 @@ __device__ __forceinline__ uint32_t zperm(uint32_t p) {
                       : w == 3u ? 0x72d236c6u : w == 4u ? 0x87271e4eu : 0x93634b1bu;
   return (word >> ((p & 3u) * 8u)) & 255u;
 }
-__device__ uint32_t zsobol_index(uint32_t morton, uint32_t dim, uint32_t logSPP) {
+__device__ __forceinline__ uint32_t zsobol_index(uint32_t morton, uint32_t dim, uint32_t logSPP) {
   uint32_t odd = logSPP & 1u;
   int digits = 8 + (int)((logSPP + 1u) >> 1);
   uint32_t result = 0;
@@ -194,7 +194,7 @@ struct Smp {
   }
   // lightCandidateRandom (rayTrace.compute.ts:251-261): the random pattern
   // discards one draw to keep its stream, the value is always the hash.
-  __device__ float candidate_random(uint32_t salt) const {
+  __device__ __forceinline__ float candidate_random(uint32_t salt) const {
     if (pattern == kPatternRandom) (void)rnd();
     uint32_t pixelID = px + py * width;
     uint32_t key = sseed(sseed(pixelID, index), seed);
@@ -204,7 +204,7 @@ struct Smp {
 };
 
 // ---------------------------------------------------------------- BSDF math
-__device__ f3 ggx_vndf(f3 view, float ax, float ay, float sx, float sy) {
+__device__ __forceinline__ f3 ggx_vndf(f3 view, float ax, float ay, float sx, float sy) {
   f3 st{ax, ay, 1.0f};
   f3 sv = normalize(st * view);
   float vz = mnf(sv.z, 1.0f);
@@ -229,7 +229,7 @@ __device__ __forceinline__ float smith_g1(f3 d, float ax, float ay) {
   return 2.0f / (1.0f + sqrtf(1.0f + tan2));
 }
 __device__ __forceinline__ float schlick5(float c) { return mtxfm::powf(clampf(1.0f - c, 0.0f, 1.0f), 5.0f); }
-__device__ float fresnel_dielectric(float incidentCos, float eta) {
+__device__ __forceinline__ float fresnel_dielectric(float incidentCos, float eta) {
   float cosI = clampf(fabsf(incidentCos), 0.0f, 1.0f);
   float sinT2 = eta * eta * mxf(0.0f, 1.0f - cosI * cosI);
   if (sinT2 >= 1.0f) return 1.0f;
@@ -238,7 +238,7 @@ __device__ float fresnel_dielectric(float incidentCos, float eta) {
   float par = (eta * cosI - cosT) / mxf(eta * cosI + cosT, 1e-8f);
   return 0.5f * (perp * perp + par * par);
 }
-__device__ f3 cosine_hemisphere(float sx, float sy) {
+__device__ __forceinline__ f3 cosine_hemisphere(float sx, float sy) {
   float x = 2.0f * sx - 1.0f, y = 2.0f * sy - 1.0f, dx = 0.0f, dy = 0.0f;
   if (!(x == 0.0f && y == 0.0f)) {
     float r, a;
@@ -299,7 +299,7 @@ __device__ __forceinline__ float4 mix4(float4 a, float4 b, float t) {
 // leaves interior footprints to the hardware sampler, whose weights carry
 // fewer fraction bits; its explicit four-tap form is the one used here for
 // every footprint.) A NaN coordinate (an infinite uv) samples at 0.
-__device__ float4 sample_map(const GpuScene &S, uint32_t index, float2 uv) {
+__device__ __forceinline__ float4 sample_map(const GpuScene &S, uint32_t index, float2 uv) {
   const GpuTexture t = S.textures[index];
   const uint32_t ms = (t.flags >> 1) & 3u, mt = (t.flags >> 3) & 3u;
   float wu = wrap_coord(uv.x * t.sx + t.ox, ms), wv = wrap_coord(uv.y * t.sy + t.oy, mt);
@@ -335,7 +335,7 @@ __device__ __forceinline__ float4 map_at(const GpuScene &S, uint32_t slot, float
 // getMaterialEmission (materialBuffer.wgsl.ts:351-372): the packed emission
 // times the emissive map; a coat weight map moves the coat tint, which the
 // packed emission then leaves out, to the sample.
-__device__ f3 material_emission(const GpuScene &S, const float *__restrict__ m, float2 uv, float2 uv1) {
+__device__ __forceinline__ f3 material_emission(const GpuScene &S, const float *__restrict__ m, float2 uv, float2 uv1) {
   f3 e{m[MTX_MAT_EMISSION], m[MTX_MAT_EMISSION + 1], m[MTX_MAT_EMISSION + 2]};
   if (const uint32_t t = map_slot(m, MTX_MAP_EMISSIVE)) e = e * map_color(S, t - 1u, map_at(S, t, uv, uv1));
   if (const uint32_t t = map_slot(m, MTX_MAP_COAT_WEIGHT)) {
@@ -374,7 +374,7 @@ __device__ __forceinline__ void rough_alpha(float r, float aniso, float &ax, flo
 // coat weight and roughness, fuzz color and roughness, specular weight and
 // color. The coverage samples multiply ma.alpha before its alpha-mode
 // resolution in load_material.
-__device__ void apply_maps(const GpuScene &S, const float *__restrict__ m, float2 uv, float2 uv1, Mat &ma) {
+__device__ __forceinline__ void apply_maps(const GpuScene &S, const float *__restrict__ m, float2 uv, float2 uv1, Mat &ma) {
   ma.emission = material_emission(S, m, uv, uv1);
   if (const uint32_t t = map_slot(m, MTX_MAP_BASE)) {
     const float4 c = map_at(S, t, uv, uv1);
@@ -405,7 +405,7 @@ __device__ void apply_maps(const GpuScene &S, const float *__restrict__ m, float
 // material (its kernels are compiled without those lobes and the maps).
 // S: the scene whose maps apply at (uv, uv1), or null.
 template <bool kFull>
-__device__ Mat load_material(const float *__restrict__ m, const float col[3], const GpuScene *S = nullptr,
+__device__ __forceinline__ Mat load_material(const float *__restrict__ m, const float col[3], const GpuScene *S = nullptr,
                              float2 uv = float2{0.0f, 0.0f}, float2 uv1 = float2{0.0f, 0.0f}) {
   Mat ma;
   ma.baseColor = f3{m[1], m[2], m[3]};
@@ -500,7 +500,7 @@ __device__ __forceinline__ float ideal_loss(const Lut &L, float ior, float a, fl
 }
 __device__ __forceinline__ float ideal_avg(const Lut &L, float ior, float a) { return L.bi(kLutDielAvg, ior_index(ior), sqrtf(a) * 31.0f); }
 __device__ __forceinline__ float ideal_ratio(const Lut &L, float ior, float a) { return L.bi(kLutRatio, ior_index(ior), sqrtf(a) * 31.0f); }
-__device__ float metal_ec(const Lut &L, float a, float c) {
+__device__ __forceinline__ float metal_ec(const Lut &L, float a, float c) {
   float rI = clampf(sqrtf(a) * 31.0f, 0.0f, 31.0f), cI = clampf(c * 31.0f, 0.0f, 31.0f);
   int r0 = (int)floorf(rI), c0 = (int)floorf(cI);
   int r1 = min(r0 + 1, 31), c1 = min(c0 + 1, 31);
@@ -508,7 +508,7 @@ __device__ float metal_ec(const Lut &L, float a, float c) {
   return mixf(mixf(L.at(c0, kLutMetal + r0), L.at(c1, kLutMetal + r0), fc),
               mixf(L.at(c0, kLutMetal + r1), L.at(c1, kLutMetal + r1), fc), fr);
 }
-__device__ float metal_avg_ec(const Lut &L, float a) {
+__device__ __forceinline__ float metal_avg_ec(const Lut &L, float a) {
   float idx = clampf(sqrtf(a) * 31.0f, 0.0f, 31.0f);
   int i0 = (int)floorf(idx);
   return mixf(L.at(i0, kLutMetalAvg), L.at(min(i0 + 1, 31), kLutMetalAvg), fractf(idx));
@@ -524,7 +524,7 @@ __device__ __forceinline__ float spec_weighted_ior(float eta, float w) {
 __device__ __forceinline__ float pbr_fresnel(float c, float rel) {
   return fabsf(rel - 1.0f) < 1e-6f ? 0.0f : fresnel_dielectric(c, rel);
 }
-__device__ f3 metal_fresnel(float c, f3 f0, f3 tint) {
+__device__ __forceinline__ f3 metal_fresnel(float c, f3 f0, f3 tint) {
   f3 schlick = mix3(f0, splat(1.0f), schlick5(c));
   if (tint.x == 1.0f && tint.y == 1.0f && tint.z == 1.0f) return schlick;
   float edgeComp = 1.0f - kEdgeCos;
@@ -533,7 +533,7 @@ __device__ f3 metal_fresnel(float c, f3 f0, f3 tint) {
   float correction = c * schlick5(c) * comp / (kEdgeCos * mtxfm::powf(edgeComp, 6.0f));
   return clamp3(schlick - correction * (edgeF - tint * edgeF), 0.0f, 1.0f);
 }
-__device__ f3 eval_diffuse(const Mat &m, f3 color, f3 v, f3 l, float comp, float &pdf) {
+__device__ __forceinline__ f3 eval_diffuse(const Mat &m, f3 color, f3 v, f3 l, float comp, float &pdf) {
   pdf = 0.0f;
   if (l.z <= 0.0f) return splat(0.0f);
   float r = m.diffuseRoughness, muI = l.z, muO = v.z;
@@ -552,14 +552,14 @@ __device__ f3 eval_diffuse(const Mat &m, f3 color, f3 v, f3 l, float comp, float
   pdf = l.z * kInvPi;
   return (single + multiple) * comp;
 }
-__device__ f3 eval_refl(float ax, float ay, f3 v, f3 l, f3 h, f3 F, float &pdf) {
+__device__ __forceinline__ f3 eval_refl(float ax, float ay, f3 v, f3 l, f3 h, f3 F, float &pdf) {
   pdf = 0.0f;
   if (l.z <= 0.0f) return splat(0.0f);
   float D = ggx_ndf(h, ax, ay), G1 = smith_g1(v, ax, ay), G2 = G1 * smith_g1(l, ax, ay);
   pdf = G1 * D / (4.0f * mxf(v.z, 1e-8f));
   return F * D * G2 / (4.0f * mxf(l.z * v.z, 1e-8f));
 }
-__device__ f3 eval_refr(float ax, float ay, float rel, f3 tint, f3 v, f3 l, f3 h, f3 F, float &pdf) {
+__device__ __forceinline__ f3 eval_refr(float ax, float ay, float rel, f3 tint, f3 v, f3 l, f3 h, f3 F, float &pdf) {
   pdf = 0.0f;
   if (l.z >= 0.0f) return splat(0.0f);
   float lh = dot(l, h), vh = dot(v, h);
@@ -577,12 +577,12 @@ __device__ __forceinline__ float avg_fresnel(float eta) {
   if (eta > 1.0f) return (eta - 1.0f) / (4.08567f + 1.00071f * eta);
   return 0.997118f + 0.1014f * eta - 0.965241f * eta * eta - 0.130607f * eta * eta * eta;
 }
-__device__ f3 metal_avg_fresnel(f3 f0, f3 tint) {
+__device__ __forceinline__ f3 metal_avg_fresnel(f3 f0, f3 tint) {
   f3 edgeF = mix3(f0, splat(1.0f), schlick5(kEdgeCos));
   f3 b = edgeF * (splat(1.0f) - tint) / (kEdgeCos * mtxfm::powf(1.0f - kEdgeCos, 6.0f));
   return clamp3(f0 + (splat(1.0f) - f0) / 21.0f - b / 126.0f, 0.0f, 1.0f);
 }
-__device__ f3 coat_passage(const Mat &m, float c) {
+__device__ __forceinline__ f3 coat_passage(const Mat &m, float c) {
   if (c <= 0.0f) return splat(1.0f);
   float rc = sqrtf(mxf(0.0f, 1.0f - (1.0f - c * c) / (m.coatIor * m.coatIor)));
   f3 passage = vpow(vmaxs(m.coatColor, 0.0f), splat(0.5f / mxf(rc, 1e-5f)));
@@ -599,7 +599,7 @@ constexpr float kSqrtTwoPi = KF(2.506628274631083);
 // albedo of the fuzz lobe, a Gaussian in the view cosine whose scale, mean
 // and offset are rational functions of the roughness. pow(z, 2) is written
 // z * z, its correctly rounded value.
-__device__ float fuzz_albedo(float viewCosine, float roughness) {
+__device__ __forceinline__ float fuzz_albedo(float viewCosine, float roughness) {
   const float x = clampf(viewCosine, 0.0f, 1.0f);
   const float y = clampf(roughness, 0.01f, 1.0f);
   const float scale = y * (0.0206607f + 1.58491f * y) / (0.0379424f + y * (1.32227f + y));
@@ -623,7 +623,7 @@ struct Prep {
   float w[LN], p[LN];
 };
 
-__device__ f3 coat_darkening(const Prep &P) {
+__device__ __forceinline__ f3 coat_darkening(const Prep &P) {
   const Mat &m = P.m;
   float diel = 1.0f - m.baseMetalness;
   float opaque = diel * (1.0f - m.transmissionWeight) * (1.0f - m.subsurfaceWeight);
@@ -653,7 +653,7 @@ __device__ __forceinline__ float thin_wall_fresnel(float f) { return 2.0f * f / 
 __device__ __forceinline__ float thin_wall_reflection(float f, float transmissionWeight) {
   return mixf(f, 2.0f * f / (1.0f + f), clampf(transmissionWeight, 0.0f, 1.0f));
 }
-__device__ f3 final_transmission_tint(const Mat &m, float incidentCos, float eta) {
+__device__ __forceinline__ f3 final_transmission_tint(const Mat &m, float incidentCos, float eta) {
   const f3 tint = m.transmissionColor;
   if (!m.thinWalled) return tint;
   const float sinI2 = mxf(0.0f, 1.0f - incidentCos * incidentCos);
@@ -664,7 +664,7 @@ __device__ f3 final_transmission_tint(const Mat &m, float incidentCos, float eta
 }
 // openpbr_eval_subsurface_boundary (openPbrBsdf.wgsl.ts:733-750): the
 // diffuse transmission into a non-thin subsurface medium.
-__device__ f3 eval_subsurface_boundary(const Mat &m, f3 v, f3 l, float &pdf) {
+__device__ __forceinline__ f3 eval_subsurface_boundary(const Mat &m, f3 v, f3 l, float &pdf) {
   pdf = 0.0f;
   if ((v.z <= 0.0f) | (l.z >= 0.0f)) return splat(0.0f);
   const float entry = fresnel_dielectric(v.z, m.relativeIor);
@@ -672,7 +672,7 @@ __device__ f3 eval_subsurface_boundary(const Mat &m, f3 v, f3 l, float &pdf) {
   return splat(1.0f - entry) * kInvPi;
 }
 
-__device__ void prepare(Prep &P, const Mat &m, f3 view, f3 normal, const Lut &L) {
+__device__ __forceinline__ void prepare(Prep &P, const Mat &m, f3 view, f3 normal, const Lut &L) {
   P.m = m;
   P.basis = make_basis(normal);
   P.v = to_local(P.basis, view);
@@ -786,7 +786,7 @@ __device__ __forceinline__ float substrate_fresnel(const Prep &P, float c, bool 
   return mixf(oF, tF, nonOpaque);
 }
 
-__device__ f3 eval_bsdf(const Prep &P, f3 lightDir, float &pdf, const Lut &L) {
+__device__ __forceinline__ f3 eval_bsdf(const Prep &P, f3 lightDir, float &pdf, const Lut &L) {
   const Mat &m = P.m;
   f3 v = P.v, l = to_local(P.basis, lightDir);
   bool reflection = l.z * v.z > 0.0f;
@@ -883,7 +883,7 @@ __device__ f3 eval_bsdf(const Prep &P, f3 lightDir, float &pdf, const Lut &L) {
   return resp * fabsf(l.z);
 }
 
-__device__ bool sample_bsdf(const Prep &P, float rx, float ry, float lobe, f3 &dir, bool &transmission) {
+__device__ __forceinline__ bool sample_bsdf(const Prep &P, float rx, float ry, float lobe, f3 &dir, bool &transmission) {
   const Mat &m = P.m;
   f3 v = P.v;
   transmission = false;
@@ -963,7 +963,7 @@ struct LSample {
 };
 
 __device__ __forceinline__ float4 env_texel(const GpuScene &S, int x, int y) { return S.env[(size_t)y * S.envW + x]; }
-__device__ f3 texture_linear(const GpuScene &S, float u, float v) {
+__device__ __forceinline__ f3 texture_linear(const GpuScene &S, float u, float v) {
   float fx = u * (float)S.envW - 0.5f, fy = v * (float)S.envH - 0.5f;
   float flx = floorf(fx), fly = floorf(fy);
   float tx = fx - flx, ty = fy - fly;
@@ -990,7 +990,7 @@ __device__ __forceinline__ float env_solid_pdf(float px, float py, float v) {
   float sinT = mtxfm::sinf(mnf(v, 1.0f - v) * kPi);
   return px * py * kInvPi2 / (2.0f * sinT);
 }
-__device__ float env_pdf(const GpuScene &S, float u, float v) {
+__device__ __forceinline__ float env_pdf(const GpuScene &S, float u, float v) {
   int x = min(max((int)(u * (float)S.envW), 0), (int)S.envW - 1);
   int y = min(max((int)(v * (float)S.envH), 0), (int)S.envH - 1);
   return env_solid_pdf(cdf_at(S, 1 + x, y).y, cdf_at(S, 0, y).y, v);
@@ -1007,7 +1007,7 @@ __device__ __forceinline__ void env_bracket(const uint16_t *guide, uint32_t bins
     hi = guide[k + 1];
   }
 }
-__device__ f3 sample_env(const GpuScene &S, float r0, float r1, float &u, float &v, float &pdf) {
+__device__ __forceinline__ f3 sample_env(const GpuScene &S, float r0, float r1, float &u, float &v, float &pdf) {
   int H = (int)S.envH, W = (int)S.envW;
   int left, right;
   env_bracket(S.envGuide, kEnvGuideRows, r0, H + 1, left, right);
@@ -1042,7 +1042,7 @@ __device__ __forceinline__ int light_type(const float *__restrict__ L) {
 }
 constexpr float kInv4Pi = KF(0.07957747154594766);
 
-__device__ void sample_rect(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
+__device__ __forceinline__ void sample_rect(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
   f3 U{L[4], L[5], L[6]}, V{L[7], L[8], L[9]}, pos{L[1], L[2], L[3]};
   f3 n = normalize(cross(U, V));
   f3 lowerLeft = pos - 0.5f * (U + V);
@@ -1061,7 +1061,7 @@ __device__ void sample_rect(const float *__restrict__ L, f3 p, float sx, float s
 // light_sample_sphere (sampleLight.wgsl.ts:10-89): a zero radius is a point
 // emitter (delta, emission = intensity / d^2); inside the sphere uniform
 // directions, outside cone sampling with the cancellation-free solid angle.
-__device__ void sample_sphere(const float *__restrict__ L, f3 p, float rx, float ry, LSample &r) {
+__device__ __forceinline__ void sample_sphere(const float *__restrict__ L, f3 p, float rx, float ry, LSample &r) {
   const f3 pos{L[1], L[2], L[3]}, E{L[10], L[11], L[12]};
   const f3 co = pos - p;
   const float cd = len(co);
@@ -1114,7 +1114,7 @@ __device__ void sample_sphere(const float *__restrict__ L, f3 p, float rx, float
 }
 // evaluateSpotEmissionMultiplier (rayTraceCore.wgsl.ts:365-378), without IES
 // profiles: hard cone at cos(outer) = v.x, smoothstep to cos(inner) = v.y.
-__device__ float spot_multiplier(const float *__restrict__ L, f3 lightToSurface) {
+__device__ __forceinline__ float spot_multiplier(const float *__restrict__ L, f3 lightToSurface) {
   const f3 axis = normalize(f3{L[4], L[5], L[6]});
   const float cosT = dot(axis, lightToSurface);
   float cone = cosT >= L[7] ? 1.0f : 0.0f;
@@ -1126,7 +1126,7 @@ __device__ float spot_multiplier(const float *__restrict__ L, f3 lightToSurface)
 }
 // light_sample_disk / light_sample_cylinder (sampleLight.wgsl.ts:163-195):
 // area sampling, pdf = d^2 / (area cos).
-__device__ void sample_area_point(const float *__restrict__ L, f3 p, f3 surf, f3 normal, LSample &r) {
+__device__ __forceinline__ void sample_area_point(const float *__restrict__ L, f3 p, f3 surf, f3 normal, LSample &r) {
   const f3 off = surf - p;
   const float d2 = dot(off, off);
   r.dist = sqrtf(d2);
@@ -1136,14 +1136,14 @@ __device__ void sample_area_point(const float *__restrict__ L, f3 p, f3 surf, f3
   r.emission = f3{L[10], L[11], L[12]};
   r.pdf = d2 / mxf(L[14] * ec, 1e-8f);
 }
-__device__ void sample_disk(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
+__device__ __forceinline__ void sample_disk(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
   const f3 U{L[4], L[5], L[6]}, V{L[7], L[8], L[9]}, pos{L[1], L[2], L[3]};
   const float rr = sqrtf(sx), phi = kTwoPi * sy;
   const mtxfm::SinCos a = mtxfm::sincosf(phi);
   const f3 surf = pos + U * (rr * a.c) + V * (rr * a.s);
   sample_area_point(L, p, surf, normalize(cross(U, V)), r);
 }
-__device__ void sample_cylinder(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
+__device__ __forceinline__ void sample_cylinder(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
   const f3 U{L[4], L[5], L[6]}, V{L[7], L[8], L[9]}, pos{L[1], L[2], L[3]};
   const f3 axis = normalize(U), r0 = normalize(V), r1 = normalize(cross(axis, r0));
   const float phi = kTwoPi * sy;
@@ -1153,7 +1153,7 @@ __device__ void sample_cylinder(const float *__restrict__ L, f3 p, float sx, flo
   sample_area_point(L, p, surf, normal, r);
 }
 // sampleAnalyticLight (sampleLight.wgsl.ts:223-253).
-__device__ void sample_analytic(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
+__device__ __forceinline__ void sample_analytic(const float *__restrict__ L, f3 p, float sx, float sy, LSample &r) {
   switch (light_type(L)) {
     case kLightRect: sample_rect(L, p, sx, sy, r); break;
     case kLightSphere: sample_sphere(L, p, sx, sy, r); break;
@@ -1180,7 +1180,7 @@ __device__ void sample_analytic(const float *__restrict__ L, f3 p, float sx, flo
 // textured scenes evaluate getMaterialEmission at the point's interpolated
 // (unscaled) UVs.
 template <bool kFull>
-__device__ void sample_emissive(const GpuScene &S, uint32_t index, f3 p, float rx, float ry, LSample &r) {
+__device__ __forceinline__ void sample_emissive(const GpuScene &S, uint32_t index, f3 p, float rx, float ry, LSample &r) {
   const float4 a = S.emissive[3 * index], b = S.emissive[3 * index + 1], c = S.emissive[3 * index + 2];
   const f3 p0 = f3of(a), p1 = f3of(b), p2 = f3of(c);
   const float sqrtU = sqrtf(rx);
@@ -1207,7 +1207,7 @@ __device__ void sample_emissive(const GpuScene &S, uint32_t index, f3 p, float r
   r.pdf = a.w * (r.dist * r.dist) / mxf(b.w * cosLight, 1e-8f);
 }
 template <bool kFull>
-__device__ void sample_light(const GpuScene &S, f3 p, float rx, float ry, float rz, uint32_t cand, uint32_t count,
+__device__ __forceinline__ void sample_light(const GpuScene &S, f3 p, float rx, float ry, float rz, uint32_t cand, uint32_t count,
                              LSample &ls) {
   uint32_t cnt = max(count, 1u);
   rz = (rz + (float)min(cand, cnt - 1u)) / (float)cnt;
@@ -1238,7 +1238,7 @@ __device__ void sample_light(const GpuScene &S, f3 p, float rx, float ry, float 
   }
 }
 // intersectSphere (intersect.wgsl.ts:924-945).
-__device__ float intersect_sphere(float rad, f3 pos, f3 ro, f3 rd) {
+__device__ __forceinline__ float intersect_sphere(float rad, f3 pos, f3 ro, f3 rd) {
   const f3 op = pos - ro;
   const float b = dot(op, rd);
   float det = b * b - dot(op, op) + rad * rad;
@@ -1251,7 +1251,7 @@ __device__ float intersect_sphere(float rad, f3 pos, f3 ro, f3 rd) {
   return kInf;
 }
 // sphereSolidAnglePdf (intersect.wgsl.ts:966-974).
-__device__ float sphere_solid_angle_pdf(f3 origin, f3 center, float radius) {
+__device__ __forceinline__ float sphere_solid_angle_pdf(f3 origin, f3 center, float radius) {
   const float cd = len(origin - center);
   if (cd <= radius) return kInv4Pi;
   const float s2 = mnf(1.0f, radius * radius / (cd * cd));
@@ -1261,7 +1261,7 @@ __device__ float sphere_solid_angle_pdf(f3 origin, f3 center, float radius) {
 // intersectLight (intersect.wgsl.ts:976-1122): distance to the analytic light
 // along a continuation ray (kInf when missed or not hittable) with the
 // light's emission and the conditional density NEE would have used.
-__device__ float intersect_light(const float *__restrict__ L, f3 ro, f3 rd, LSample &ls) {
+__device__ __forceinline__ float intersect_light(const float *__restrict__ L, f3 ro, f3 rd, LSample &ls) {
   ls.pdf = 0.0f;
   ls.emission = splat(0.0f);
   ls.isDelta = false;
@@ -1379,7 +1379,7 @@ struct Surf {
 // getMatNormal (materialBuffer.wgsl.ts:377-415): the normal map's tangent-
 // space normal in the cotangent frame of UV0 (dp1 = p0 - p2, dp2 = p1 - p2,
 // duv the raw vertex UV differences), object space.
-__device__ f3 mapped_normal(const GpuScene &S, uint32_t slot, const float *__restrict__ m, float2 uv, f3 normal,
+__device__ __forceinline__ f3 mapped_normal(const GpuScene &S, uint32_t slot, const float *__restrict__ m, float2 uv, f3 normal,
                             f3 dp1, f3 dp2, float2 duv1, float2 duv2) {
   const f3 dp2perp = cross(dp2, normal), dp1perp = cross(normal, dp1);
   f3 dpdu = dp2perp * duv1.x + dp1perp * duv2.x;
@@ -1404,10 +1404,10 @@ __device__ f3 mapped_normal(const GpuScene &S, uint32_t slot, const float *__res
 // 1539-1601). kFull: textured scenes also interpolate the UV sets, scale
 // them by the material's UV scale and apply its normal map.
 template <bool kFull = true>
-__device__ void complete_surface(const GpuScene &S, const TraceHit &h, Surf &si) {
+__device__ __forceinline__ void complete_surface(const GpuScene &S, const TraceHit &h, Surf &si) {
   const ShadeSlot &sh = S.shade[h.slot];
-  const InstSlot &is = S.accel->slots[h.slot];
-  const TriRec r = is.tris[h.tri];
+  const InstSlot &is = global_ptr(S.accel->slots)[h.slot];
+  const TriRec r = global_ptr(is.tris)[h.tri];
   uint32_t src = (uint32_t)fint(r.v0.w);
   uint32_t i0 = sh.indices[src * 3], i1 = sh.indices[src * 3 + 1], i2 = sh.indices[src * 3 + 2];
   f3 p0 = f3of(r.v0), p1 = f3of(r.v1), p2 = f3of(r.v2);
@@ -1479,7 +1479,7 @@ __device__ void complete_surface(const GpuScene &S, const TraceHit &h, Surf &si)
 // is coverage, times the alpha map's g; both maps are sampled at UV0 * the
 // material's UV scale (the any-hit test reads no UV1 set), and the triangle
 // occludes when the coverage reaches the cutoff.
-__device__ bool alpha_covers(const GpuScene &S, int32_t slot, int32_t tri, f3 b) {
+__device__ __forceinline__ bool alpha_covers(const GpuScene &S, int32_t slot, int32_t tri, f3 b) {
   const ShadeSlot &sh = S.shade[slot];
   const float *__restrict__ m = S.materials + (size_t)sh.material * MTX_MATERIAL_FLOATS;
   float alpha = m[MTX_MAT_OPACITY];
@@ -1489,7 +1489,7 @@ __device__ bool alpha_covers(const GpuScene &S, int32_t slot, int32_t tri, f3 b)
     if (base | amap) {
       float2 uv{0.0f, 0.0f};
       if (sh.uvs != nullptr) {
-        const TriRec r = S.accel->slots[slot].tris[tri];
+        const TriRec r = global_ptr(S.accel->slots)[slot].tris[tri];
         const uint32_t src = (uint32_t)fint(r.v0.w);
         const uint32_t i0 = sh.indices[src * 3], i1 = sh.indices[src * 3 + 1], i2 = sh.indices[src * 3 + 2];
         const float2 t0{sh.uvs[i0 * 2], sh.uvs[i0 * 2 + 1]}, t1{sh.uvs[i1 * 2], sh.uvs[i1 * 2 + 1]};
@@ -1582,7 +1582,7 @@ __device__ __forceinline__ void sample_circle(float ux, float uy, float &cx, flo
 // positive aperture, the thin lens: focus plane perpendicular to the view
 // direction at the focus distance, lens point = aperture *
 // sampleCircle(CAMERA_LENS sample).
-__device__ void init_path(const RenderParams &P, const Smp &smp, PathRegs &pr) {
+__device__ __forceinline__ void init_path(const RenderParams &P, const Smp &smp, PathRegs &pr) {
   const float Wf = (float)P.width, Hf = (float)P.height;
   float uvx = ((float)smp.px + 0.5f) / Wf, uvy = ((float)smp.py + 0.5f) / Hf;
   float jx, jy;
@@ -1646,8 +1646,12 @@ __device__ __forceinline__ int path_depth(uint32_t flags) { return (int)(flags >
 // kFull = false compiles the event for scenes without fuzz, subsurface and
 // thin-walled materials and without the random pattern; the launcher picks
 // it only then, so it computes the same values as the full form.
+// Everything here is inlined: called out of line, the event and the lobes took
+// the scene, the material and the path through scratch memory with flat loads
+// (469 of them in the full form; shading of the textured room 2.85 -> 1.91 ms
+// a 381 x 277 x 12 frame).
 template <bool kFull = true>
-__device__ bool shade_event(const GpuScene &S, const RenderParams &P, const Lut &L, PathRegs &pr, const TraceHit &h,
+__device__ __forceinline__ bool shade_event(const GpuScene &S, const RenderParams &P, const Lut &L, PathRegs &pr, const TraceHit &h,
                             int event, Smp &smp, ShadowReq &sr) {
   if (!kFull && smp.pattern == kPatternRandom) __builtin_unreachable();
   sr.valid = false;

@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
         const int slot = W.hitB[p].x;
         const AccelView *av = job_of<kMulti>(L, W, p).scene.accel;
         cls = slot < 0 ? kShadeMiss
-                       : (int)((fbits(av->slots[slot].c3.w) & kSlotClassMask) >> kSlotClassShift);
+                       : (int)((fbits(global_ptr(av->slots)[slot].c3.w) & kSlotClassMask) >> kSlotClassShift);
       }
 #pragma unroll
       for (int c = 0; c < kShadeClasses; c++) {
@@ -266,8 +266,8 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
         h.t = ha.x;
         h.bary = f3{ha.y, ha.z, ha.w};
         // The traversal's object-space hit data, recomputed from the same inputs.
-        const InstSlot &is = S.accel->slots[h.slot];
-        const TriRec r = is.tris[h.tri];
+        const InstSlot &is = global_ptr(S.accel->slots)[h.slot];
+        const TriRec r = global_ptr(is.tris)[h.tri];
         const f3 p0 = f3of(r.v0), p1 = f3of(r.v1), p2 = f3of(r.v2);
         h.normal = normalize(cross(p1 - p0, p2 - p0));
         const Affine w2l{f3of(is.c0), f3of(is.c1), f3of(is.c2), f3of(is.c3)};
