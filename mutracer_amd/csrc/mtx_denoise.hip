@@ -34,6 +34,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <mutex>
+#include <thread>
 
 #include "../../include/mtx_fmath.h"
 #include "mtx_registry.h"
@@ -686,8 +687,11 @@ struct DenoiserObj {
   // Prefilters of the albedo and normal guides (clean-auxiliary models).
   std::shared_ptr<DenoiserObj> auxAlbedo, auxNormal;
   hipStream_t stream = nullptr;
+  hipStream_t copies[2] = {nullptr, nullptr};  // beside `stream` for large host copies, made by the first
   std::mutex busy;
   ~DenoiserObj() {
+    for (hipStream_t c : copies)
+      if (c) (void)hipStreamDestroy(c);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -921,6 +925,51 @@ static void download_layer(DenoiserObj &D, int i, int H, int W, float *out, hipS
     for (int c = 0; c < co; c++) out[p * co + c] = D.bf16 ? bf16_to_f32(h[p * cs + c]) : f16_to_f32(h[p * cs + c]);
 }
 
+// Three host <-> device copies, done when it returns. A copy of pageable
+// memory goes at the pace of the thread that issues it, so large ones take a
+// thread and a stream each (blocking streams, ordered after earlier
+// null-stream work as D.stream is). A 1080p run (100 MB in, 33 MB out) took
+// 13.9 ms; with the result straight into the caller's buffer 6.5, with the
+// uploads on threads 5.8, with the download too 4.8.
+struct HostCopy {
+  void *dst;
+  const void *src;
+  size_t bytes;
+  hipMemcpyKind kind;
+};
+constexpr size_t kThreadedCopyBytes = 4u << 20;  // 509 x 287 (7 MB in): 0.73 -> 0.64 ms; small runs need no threads
+static void host_copies(DenoiserObj &D, const HostCopy (&c)[3]) {
+  if (c[0].bytes + c[1].bytes + c[2].bytes < kThreadedCopyBytes) {
+    for (const HostCopy &k : c)
+      if (k.bytes) MTX_HIP(hipMemcpyAsync(k.dst, k.src, k.bytes, k.kind, D.stream));
+    MTX_HIP(hipStreamSynchronize(D.stream));
+    return;
+  }
+  int dev = 0;
+  MTX_HIP(hipGetDevice(&dev));
+  for (hipStream_t &s : D.copies)
+    if (!s) MTX_HIP(hipStreamCreate(&s));
+  hipError_t err[3] = {hipSuccess, hipSuccess, hipSuccess};
+  auto copy = [&](int k) {
+    if (!c[k].bytes) return;
+    const hipStream_t st = k ? D.copies[k - 1] : D.stream;
+    err[k] = hipSetDevice(dev);
+    if (err[k] == hipSuccess) err[k] = hipMemcpyAsync(c[k].dst, c[k].src, c[k].bytes, c[k].kind, st);
+    if (err[k] == hipSuccess) err[k] = hipStreamSynchronize(st);
+  };
+  std::thread t[2];
+  try {
+    for (int k = 0; k < 2; k++) t[k] = std::thread(copy, k + 1);
+  } catch (const std::exception &) {  // no thread to be had: the remaining copies run here
+  }
+  copy(0);
+  for (int k = 0; k < 2; k++) {
+    if (t[k].joinable()) t[k].join();
+    else copy(k + 1);
+  }
+  for (hipError_t e : err) MTX_HIP(e);
+}
+
 // One image through a network, tile by tile: tiles of max_tile pixels (0 =
 // the whole image), each run on its region grown by `overlap` pixels on
 // every side (clipped to the image, padded to a multiple of 16) and written
@@ -1144,9 +1193,10 @@ int32_t mtx_denoiser_run(mtx_handle handle, uint32_t width, uint32_t height, con
       D->ioPixels = n;
     }
     hipStream_t s = D->stream;
-    D->io[0].upload(reinterpret_cast<const float4 *>(color), n, s);
-    D->io[1].upload(reinterpret_cast<const float4 *>(albedo), n, s);
-    D->io[2].upload(reinterpret_cast<const float4 *>(normal), n, s);
+    const size_t bytes = n * sizeof(float4);
+    host_copies(*D, {{D->io[0].ptr, color, bytes, hipMemcpyHostToDevice},
+                     {D->io[1].ptr, albedo, bytes, hipMemcpyHostToDevice},
+                     {D->io[2].ptr, normal, bytes, hipMemcpyHostToDevice}});
     const float4 *guideA = D->io[1].ptr, *guideN = D->io[2].ptr;
     if (D->auxAlbedo) {
       // Clean auxiliary guides (WGPURenderingPipeline.ts:1352-1440,
@@ -1161,8 +1211,13 @@ int32_t mtx_denoiser_run(mtx_handle handle, uint32_t width, uint32_t height, con
     denoise_image(*D, D->maxTile, D->overlap, D->io[0].ptr, guideA, guideN, (int)width, (int)height, kNetBeauty,
                   D->io[3].ptr, s);
     MTX_HIP(hipGetLastError());
-    std::vector<float4> res = D->io[3].to_host(n, s);  // no partial result on failure: copy after success
-    std::memcpy(output, res.data(), n * sizeof(float4));
+    MTX_HIP(hipStreamSynchronize(s));  // the caller's buffer is written only after the run has succeeded
+    const size_t part = n / 3;
+    float4 *out = reinterpret_cast<float4 *>(output);
+    host_copies(*D, {{out, D->io[3].ptr, part * sizeof(float4), hipMemcpyDeviceToHost},
+                     {out + part, D->io[3].ptr + part, part * sizeof(float4), hipMemcpyDeviceToHost},
+                     {out + 2 * part, D->io[3].ptr + 2 * part, (n - 2 * part) * sizeof(float4),
+                      hipMemcpyDeviceToHost}});
     return MTX_OK;
   } catch (const Error &e) {
     set_error(err, cap, e.what());

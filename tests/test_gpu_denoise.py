@@ -291,6 +291,31 @@ def test_tiles(net):
     assert _rel(out[..., :3], ref[..., :3]) <= RUN_TOL["fp16"]
 
 
+@pytest.mark.parametrize("h,w", [(273, 320), (274, 320)])
+def test_run_host_copies(net, h, w):
+    """Images on both sides of the size from which a run's host copies go out
+    on threads (4 MiB of inputs, 87381 pixels; 274 x 320 has a download of
+    unequal thirds): tiled runs equal the untiled runs of their regions,
+    which are below that size, stitched bit for bit, twice."""
+    denoise, _ = net
+    d = denoise.Denoiser("fp16")
+    d.set_input_scale(0.8)
+    color, albedo, normal = _images(h, w, seed=14)
+    images = (color, normal, albedo)
+    expect = np.zeros((h, w, 4), np.float32)
+    t, ov = 160, 16
+    for ty in range(0, h, t):
+        for tx in range(0, w, t):
+            y0, y1, x0, x1 = max(0, ty - ov), min(h, ty + t + ov), max(0, tx - ov), min(w, tx + t + ov)
+            r = d.run(*[np.ascontiguousarray(a[y0:y1, x0:x1]) for a in images])
+            expect[ty:ty + t, tx:tx + t] = r[ty - y0:ty - y0 + t, tx - x0:tx - x0 + t]
+    d.set_tiles(t, ov)
+    for _ in range(2):
+        out = d.run(*images)
+        assert np.array_equal(out, expect)
+        assert np.array_equal(out[..., 3], images[0][..., 3])
+
+
 def test_denoiser_validation(net):
     from mutracer_amd import abi
     denoise, _ = net
