@@ -528,12 +528,25 @@ struct SmallBlockArrays {
   uint32_t ltmp[kSmall], X[kSmall], Z[kSmall], rk[kSmall];
   uint32_t kmin[3 * kMaxBins * 3], kmax[3 * kMaxBins * 3], cnt[3 * kMaxBins];
 };
+// Nodes of at most kRowNode primitives, with at most kRowNode bins, are split
+// four at a time, one to a row of 16 lanes: most nodes of a tree are that
+// small, the kernel is bound by vector instruction issue, and a wave with one
+// of them has work for a fifth of its lanes. 1M triangles in 8 bins: the
+// kernel takes 9.8 -> 4.1 ms, the build with its scene 19.1 -> 13.1 ms. (LDS
+// sized by the bins for a fourth workgroup per CU: 4.0 at the same three,
+// 4.1 at four, 16 registers spilled; twice the id atomics: the same time.)
+constexpr int kRowNode = 16, kRows = 64 / kRowNode;
+// A wave's pending nodes hold two primitives or more each and are parts of
+// one queued node, beside at most kRows - 1 left of earlier ones.
+constexpr int kWaveStack = kWaveNode / 2 + kRows;
 struct SmallWaveArrays {
+  // one node's bins, or those of kRows nodes with at most kRowNode bins each
   uint32_t kmin[3 * kMaxBins * 3], kmax[3 * kMaxBins * 3], cnt[3 * kMaxBins];
   uint32_t X[kWaveNode], Z[kWaveNode], tmp[kWaveNode];
-  uint32_t stack[kWaveNode + 2];  // pending node ids and their records
-  BNode snode[kWaveNode + 2];
+  uint32_t stack[kWaveStack];  // pending node ids and their records: wide from the front, row nodes from the back
+  BNode snode[kWaveStack];
 };
+static_assert(kRows * kRowNode <= kMaxBins, "a wave's bin arrays hold four row nodes' bins");
 
 // Cross-lane steps through DPP (gfx9 row shifts and row broadcasts, no LDS
 // traffic); a lane without a source keeps `old`.
@@ -571,6 +584,35 @@ __device__ __forceinline__ uint32_t scan_add(uint32_t v, bool seg64) {
   v += dpp_u<0x142, 0xa>(0u, v);
   if (seg64) v += dpp_u<0x143, 0xc>(0u, v);
   return v;
+}
+// The same over rows of 16 lanes.
+template <bool kMax>
+__device__ __forceinline__ float row_minmax(float v) {
+  const float nt = kMax ? -INFINITY : INFINITY;
+  float e;
+  e = dpp_f<0x111, 0xf>(nt, v); v = kMax ? (v > e ? v : e) : (v < e ? v : e);
+  e = dpp_f<0x112, 0xf>(nt, v); v = kMax ? (v > e ? v : e) : (v < e ? v : e);
+  e = dpp_f<0x114, 0xf>(nt, v); v = kMax ? (v > e ? v : e) : (v < e ? v : e);
+  e = dpp_f<0x118, 0xf>(nt, v); v = kMax ? (v > e ? v : e) : (v < e ? v : e);
+  return v;
+}
+__device__ __forceinline__ uint32_t row_add(uint32_t v) {
+  v += dpp_u<0x111, 0xf>(0u, v);
+  v += dpp_u<0x112, 0xf>(0u, v);
+  v += dpp_u<0x114, 0xf>(0u, v);
+  v += dpp_u<0x118, 0xf>(0u, v);
+  return v;
+}
+// One step of a minimum over a row: the lower (cost, index) of this lane's and
+// the one kShift lanes round the row; shifts of 8, 4, 2 and 1 reach all lanes.
+template <int kShift>
+__device__ __forceinline__ void row_least(double &cost, int &idx) {
+  const unsigned long long u = __builtin_bit_cast(unsigned long long, cost);
+  const uint32_t lo = dpp_u<0x120 + kShift, 0xf>((uint32_t)u, (uint32_t)u);
+  const uint32_t hi = dpp_u<0x120 + kShift, 0xf>((uint32_t)(u >> 32), (uint32_t)(u >> 32));
+  const double oc = __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+  const int oi = (int)dpp_u<0x120 + kShift, 0xf>((uint32_t)idx, (uint32_t)idx);
+  if (oc < cost || (oc == cost && oi < idx)) { cost = oc; idx = oi; }
 }
 __device__ __forceinline__ float readlane_f(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -673,6 +715,83 @@ __device__ __forceinline__ bool sah_split_wave(const uint32_t *kmin, const uint3
   return true;
 }
 
+// sah_split_wave for four nodes at once, one to a row of 16 lanes, bins <= 16:
+// lane b of the row holds bin b, the axes follow one another, and the scans,
+// the choice and the tie rules are the same within the row. `act` is the same
+// in a row; rows without a node run along. Returns whether the row's node
+// splits, the same on each of its lanes. Every lane of the wave calls it.
+__device__ __forceinline__ bool sah_split_row(const uint32_t *kmin, const uint32_t *kmax, const uint32_t *cnt,
+                                              int32_t bins, const NodeFrame &f, const double *minDim,
+                                              uint32_t nodePrims, bool act, Split &out) {
+  const int lane = threadIdx.x & 63, b = lane & (kRowNode - 1), row0 = lane - b;
+  const bool isBin = b < bins;
+  const int src = row0 + (b < bins - 1 ? bins - 2 - b : 0);
+  double bestCost = INFINITY;
+  int bestIdx = 0x7fffffff;
+#pragma unroll
+  for (int axis = 0; axis < 3; axis++) {
+    const bool ok = act && f.extent[axis] > minDim[axis];
+    if (!__any(ok)) continue;
+    const bool inb = ok && isBin;
+    const int fb = axis * bins + (isBin ? b : 0), rb = axis * bins + (isBin ? bins - 1 - b : 0);
+    const uint32_t cf = inb ? cnt[fb] : 0u, cr = inb ? cnt[rb] : 0u;
+    float lmn[3], lmx[3], rmn[3], rmx[3];
+    for (int k = 0; k < 3; k++) {
+      lmn[k] = cf ? unkey(kmin[fb * 3 + k]) : INFINITY;
+      lmx[k] = cf ? unkey(kmax[fb * 3 + k]) : -INFINITY;
+      rmn[k] = cr ? unkey(kmin[rb * 3 + k]) : INFINITY;
+      rmx[k] = cr ? unkey(kmax[rb * 3 + k]) : -INFINITY;
+    }
+    const uint32_t lc = row_add(cf), rcr = row_add(cr);
+    for (int k = 0; k < 3; k++) {
+      lmn[k] = row_minmax<false>(lmn[k]);
+      lmx[k] = row_minmax<true>(lmx[k]);
+      rmn[k] = row_minmax<false>(rmn[k]);
+      rmx[k] = row_minmax<true>(rmx[k]);
+    }
+    const uint32_t rightN = __shfl(rcr, src);
+    float sr[6];
+    for (int k = 0; k < 3; k++) { sr[k] = __shfl(rmn[k], src); sr[3 + k] = __shfl(rmx[k], src); }
+    if (ok && b < bins - 1) {
+      double L[6], R[6];
+      for (int k = 0; k < 3; k++) {
+        L[k] = (double)lmn[k] < kFar ? (double)lmn[k] : kFar;
+        L[3 + k] = (double)lmx[k] > -kFar ? (double)lmx[k] : -kFar;
+        R[k] = (double)sr[k] < kFar ? (double)sr[k] : kFar;
+        R[3 + k] = (double)sr[3 + k] > -kFar ? (double)sr[3 + k] : -kFar;
+      }
+      const double lx = L[3] - L[0], ly = L[4] - L[1], lz = L[5] - L[2];
+      const double rx = R[3] - R[0], ry = R[4] - R[1], rz = R[5] - R[2];
+      const double lcost = lc == 0 ? kFar : (lx * ly + ly * lz + lz * lx) * (double)lc;
+      const double rcost = rightN == 0 ? kFar : (rx * ry + ry * rz + rz * rx) * (double)rightN;
+      const double cost = (lcost + rcost) + 0.0;
+      if (cost < kFar && cost < bestCost) { bestCost = cost; bestIdx = axis * 64 + b; }
+    }
+  }
+  row_least<8>(bestCost, bestIdx);
+  row_least<4>(bestCost, bestIdx);
+  row_least<2>(bestCost, bestIdx);
+  row_least<1>(bestCost, bestIdx);
+  const double splitCost = 1.0 + 1.0 * (bestIdx != 0x7fffffff ? bestCost : kFar) / f.area;
+  const bool split = act && splitCost < (double)nodePrims * 1.0 && bestIdx != 0x7fffffff;
+  out.axis = split ? bestIdx >> 6 : 0;
+  out.pos = split ? bestIdx & 63 : 0;
+  const float farF = (float)kFar;
+  const int bb = out.axis * bins + (isBin ? b : 0);
+  const bool filled = split && isBin && cnt[bb] != 0;
+  for (int sd = 0; sd < 2; sd++) {
+    const bool mine = filled && (sd == 0 ? b <= out.pos : b > out.pos);
+    const int at = row0 + (sd == 0 ? out.pos : bins - 1);
+    for (int k = 0; k < 3; k++) {
+      const float vmn = __shfl(row_minmax<false>(mine ? unkey(kmin[bb * 3 + k]) : INFINITY), at);
+      const float vmx = __shfl(row_minmax<true>(mine ? unkey(kmax[bb * 3 + k]) : -INFINITY), at);
+      out.lo[sd][k] = (double)vmn < (double)farF ? vmn : farF;
+      out.hi[sd][k] = (double)vmx > (double)-farF ? vmx : -farF;
+    }
+  }
+  return split;
+}
+
 // One wave per big node of the level: its split from the level's bins (the
 // wave sweep, with the sequential fold's choice and tie rules).
 __global__ void __launch_bounds__(256) k_sweep(BigState *__restrict__ big, const uint32_t *__restrict__ nbp,
@@ -701,12 +820,11 @@ __global__ void __launch_bounds__(256) k_sweep(BigState *__restrict__ big, const
   if ((threadIdx.x & 63) == 0) big[b] = s;
 }
 
-// Writes the two children of `parent` (split at totalL), returns the first
-// child's index and, when `out` is given, the two records; one lane only.
-__device__ uint32_t emit_children(BNode *__restrict__ nodes, uint32_t *__restrict__ counter, uint32_t parentId,
-                                  const BNode &parent, const Split &split, uint32_t totalL, uint32_t totalR,
-                                  BNode *out = nullptr) {
-  const uint32_t c = atomicAdd(counter, 2u);
+// Writes the two children of `parent` (split at totalL) as nodes c and c + 1
+// and, when `out` is given, to it; one lane per parent.
+__device__ __forceinline__ void emit_children(BNode *__restrict__ nodes, uint32_t c, uint32_t parentId,
+                                              const BNode &parent, const Split &split, uint32_t totalL,
+                                              uint32_t totalR, BNode *out = nullptr) {
   for (int side = 0; side < 2; side++) {
     BNode ch{};
     for (int k = 0; k < 3; k++) { ch.lo[k] = split.lo[side][k]; ch.hi[k] = split.hi[side][k]; }
@@ -721,7 +839,6 @@ __device__ uint32_t emit_children(BNode *__restrict__ nodes, uint32_t *__restric
   nd.leftFirst = c;
   nd.primCount = 0;
   nodes[parentId] = nd;
-  return c;
 }
 
 __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *__restrict__ tasks, int32_t bins) {
@@ -850,7 +967,8 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
       __syncthreads();
       for (uint32_t e = threadIdx.x; e < n; e += blockDim.x) lp[first + e] = ltmp[e];
       if (threadIdx.x == 0) {
-        const uint32_t c = emit_children(nodes, counter, curNode, cur, split, totalL, totalR);
+        const uint32_t c = atomicAdd(counter, 2u);
+        emit_children(nodes, c, curNode, cur, split, totalL, totalR);
         const uint32_t count[2] = {totalL, totalR};
         for (int side = 1; side >= 0; side--) {
           if (count[side] > (uint32_t)kWaveNode) stack[sp++] = c + side;
@@ -860,29 +978,40 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
     }
   }
   // Phase 2: each wave takes queued nodes and splits them and their
-  // descendants on its own.
+  // descendants on its own: nodes above rowNode primitives one at a time, then
+  // the others four at a time; a wave with fewer than four of these and no
+  // wider node takes the next queued one first.
   __syncthreads();
   __threadfence_block();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   SmallWaveArrays &W = sh.w[wv];
+  const uint32_t rowNode = bins <= kRowNode ? (uint32_t)kRowNode : 0u;
+  const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
+  int wide = 0, small = 0;  // pending nodes of each kind
+  bool more = true;
+  // A node's place among the pending ones; a single primitive stays a leaf.
+  auto place = [&](uint32_t n) -> int { return n > rowNode ? wide++ : kWaveStack - 1 - small++; };
   while (true) {
-    uint32_t item = 0;
-    if (lane == 0) item = atomicAdd(&qHead, 1u);
-    item = __shfl(item, 0);
-    if (item >= qCount) break;
-    if (lane == 0) {
-      W.stack[0] = queue[item];
-      W.snode[0] = nodes[queue[item]];
+    if (more && wide == 0 && small < kRows) {
+      uint32_t item = 0;
+      if (lane == 0) item = atomicAdd(&qHead, 1u);
+      item = __shfl(item, 0);
+      if (item >= qCount) { more = false; continue; }
+      const uint32_t id = queue[item], n = nodes[id].primCount;
+      if (n > 1) {
+        const int at = place(n);
+        if (lane == 0) { W.stack[at] = id; W.snode[at] = nodes[id]; }
+        wave_sync();
+      }
+      continue;
     }
-    int wsp = 1;
-    wave_sync();
-    while (wsp > 0) {
-      --wsp;
-      const uint32_t nodeId = W.stack[wsp];
-      const BNode nd = W.snode[wsp];
+    if (wide > 0) {
+      --wide;
+      const uint32_t nodeId = W.stack[wide];
+      const BNode nd = W.snode[wide];
       const uint32_t n = nd.primCount, first = nd.leftFirst - base;
       const NodeFrame f = node_frame(nd.lo, nd.hi, bins, minDim);
-      if ((f.area == 0.0) || (n == 1)) continue;
+      if (f.area == 0.0) continue;
       for (int i = lane; i < 3 * bins * 3; i += 64) { W.kmin[i] = 0xffffffffu; W.kmax[i] = 0u; }
       for (int i = lane; i < 3 * bins; i += 64) W.cnt[i] = 0;
       wave_sync();
@@ -914,7 +1043,6 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
         r = bin_of(val, pick3(f.nMin, sp2.axis), pick3(f.scale, sp2.axis), bins) > sp2.pos;
       }
       const unsigned long long rmask = __ballot(r);
-      const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
       const uint32_t ex = (uint32_t)__popcll(rmask & below), nR = (uint32_t)__popcll(rmask);
       const uint32_t nL = n - nR;
       uint32_t rank = 0;
@@ -927,17 +1055,90 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
       if (live) W.tmp[partition_dest(lane, r, rank, Pw, n, nR, W.X, W.Z)] = p;
       wave_sync();
       if (live) lp[first + lane] = W.tmp[lane];
+      const int atR = nR > 1 ? place(nR) : -1, atL = nL > 1 ? place(nL) : -1;
       if (lane == 0) {
         BNode ch[2];
-        const uint32_t c0 = emit_children(nodes, counter, nodeId, nd, sp2, nL, nR, ch);
-        W.stack[wsp] = c0 + 1;
-        W.snode[wsp] = ch[1];
-        W.stack[wsp + 1] = c0;
-        W.snode[wsp + 1] = ch[0];
+        const uint32_t c0 = atomicAdd(counter, 2u);
+        emit_children(nodes, c0, nodeId, nd, sp2, nL, nR, ch);
+        if (atR >= 0) { W.stack[atR] = c0 + 1; W.snode[atR] = ch[1]; }
+        if (atL >= 0) { W.stack[atL] = c0; W.snode[atL] = ch[0]; }
       }
-      wsp += 2;
       wave_sync();
+      continue;
     }
+    if (small == 0) break;
+    // Up to four nodes, one to a row.
+    const int row = lane / kRowNode, b = lane & (kRowNode - 1), row0 = lane - b;
+    const bool valid = row < small;
+    const int slot = kWaveStack - (valid ? small - row : small);
+    small -= min(small, kRows);
+    const uint32_t nodeId = W.stack[slot];
+    const BNode nd = W.snode[slot];
+    const uint32_t n = valid ? nd.primCount : 0u, first = nd.leftFirst - base;
+    const NodeFrame f = node_frame(nd.lo, nd.hi, bins, minDim);
+    const bool act = valid && !(f.area == 0.0);
+    for (int i = lane; i < kRows * 3 * bins * 3; i += 64) { W.kmin[i] = 0xffffffffu; W.kmax[i] = 0u; }
+    for (int i = lane; i < kRows * 3 * bins; i += 64) W.cnt[i] = 0;
+    wave_sync();
+    uint32_t *const rmin = W.kmin + row * 9 * bins, *const rmax = W.kmax + row * 9 * bins,
+                    *const rcnt = W.cnt + row * 3 * bins;
+    const bool live = act && (uint32_t)b < n;
+    const uint32_t p = live ? lp[first + b] : 0u;
+    float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (live) {
+      c = cen[p];
+      const float4 lo = plo[p], hi = phi[p];
+      const float cc[3] = {c.x, c.y, c.z}, mn[3] = {lo.x, lo.y, lo.z}, mx[3] = {hi.x, hi.y, hi.z};
+      for (int ax = 0; ax < 3; ax++) {
+        const int bin = ax * bins + bin_of(cc[ax], f.nMin[ax], f.scale[ax], bins);
+        atomicAdd(&rcnt[bin], 1u);
+        for (int k = 0; k < 3; k++) {
+          atomicMin(&rmin[bin * 3 + k], fkey(mn[k]));
+          atomicMax(&rmax[bin * 3 + k], fkey(mx[k]));
+        }
+      }
+    }
+    wave_sync();
+    Split sp2;
+    const bool cuts = sah_split_row(rmin, rmax, rcnt, bins, f, minDim, n, act, sp2);
+    const bool moves = cuts && live;
+    bool r = false;
+    if (moves) {
+      const float val = sp2.axis == 0 ? c.x : (sp2.axis == 1 ? c.y : c.z);
+      r = bin_of(val, pick3(f.nMin, sp2.axis), pick3(f.scale, sp2.axis), bins) > sp2.pos;
+    }
+    const uint32_t rmask = (uint32_t)(__ballot(r) >> row0) & 0xffffu;
+    const uint32_t ex = (uint32_t)__popc(rmask & ((1u << b) - 1u)), nR = (uint32_t)__popc(rmask), nL = n - nR;
+    uint32_t *const rX = W.X + row0, *const rZ = W.Z + row0;
+    uint32_t rank = 0;
+    if (moves) {
+      if (r) { rX[ex] = b; rank = ex; }
+      else { rank = nL - ((uint32_t)b - ex) - 1; rZ[rank] = b; }
+    }
+    wave_sync();
+    const uint32_t Pr =
+        (uint32_t)__popc((uint32_t)(__ballot(moves && r && rank < nL && (uint32_t)b < rZ[rank]) >> row0) & 0xffffu);
+    if (moves) W.tmp[row0 + partition_dest(b, r, rank, Pr, n, nR, rX, rZ)] = p;
+    wave_sync();
+    if (moves) lp[first + b] = W.tmp[lane];
+    // The children's ids for all rows at once, and their places.
+    const bool leader = cuts && b == 0;
+    const unsigned long long lead = __ballot(leader), pushL = __ballot(leader && nL > 1),
+                             pushR = __ballot(leader && nR > 1);
+    if (lead) {
+      uint32_t c0 = 0;
+      if (lane == 0) c0 = atomicAdd(counter, 2u * (uint32_t)__popcll(lead));
+      c0 = __shfl(c0, 0) + 2u * (uint32_t)__popcll(lead & below);
+      if (leader) {
+        BNode ch[2];
+        emit_children(nodes, c0, nodeId, nd, sp2, nL, nR, ch);
+        int at = kWaveStack - 1 - small - __popcll(pushL & below) - __popcll(pushR & below);
+        if (nR > 1) { W.stack[at] = c0 + 1; W.snode[at] = ch[1]; at--; }
+        if (nL > 1) { W.stack[at] = c0; W.snode[at] = ch[0]; }
+      }
+      small += __popcll(pushL) + __popcll(pushR);
+    }
+    wave_sync();
   }
   __syncthreads();
   for (uint32_t e = threadIdx.x; e < total; e += blockDim.x) prim[base + e] = lp[e];

@@ -63,6 +63,30 @@ def test_blas_bit_exact(orc, mtx, case, bins):
     assert info["max_leaf"] == ref["max_leaf"]
 
 
+@pytest.mark.parametrize("bins", [2, 8, 15, 16, 17])
+@pytest.mark.parametrize("n", [2, 3, 15, 16, 17, 33, 63, 64, 65, 130, 1023, 1024, 1025, 1100])
+def test_blas_small_nodes_bit_exact(orc, mtx, n, bins):
+    """Trees around the sizes where a node changes hands: 16 primitives (four
+    nodes to a wave, up to 16 bins), 64 (a node to a wave), 1024 (a subtree to
+    a workgroup). Half of the triangles lie on a line of shared centres, two
+    thirds of these at one point with zeros of both signs, so that ties,
+    axes without extent and leaves of several primitives occur at every
+    level."""
+    rng = np.random.default_rng(n * 31 + bins)
+    tri = rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.05, (n, 3, 3))
+    flat = np.arange(n) % 2 == 0
+    tri[flat] = np.round(tri[flat] * 4) / 4 * np.array([1.0, 0.0, -0.0])
+    point = np.arange(n) % 3 == 0
+    tri[flat & point] = np.array([[-0.0, 0.0, 0.0], [0.5, -0.0, 0.0], [0.0, 0.5, -0.0]])
+    pos, idx = tri.reshape(-1, 3).astype(np.float32), np.arange(3 * n, dtype=np.uint32)
+    ref = orc.build_blas(pos, idx, bins)
+    b = mtx.Blas(pos, idx, bins)
+    words, src = b.export()
+    assert np.array_equal(words, ref["words"])
+    assert np.array_equal(src, ref["source_of_record"])
+    assert b.info()["max_depth"] == ref["max_depth"] and b.info()["max_leaf"] == ref["max_leaf"]
+
+
 def test_blas_device_input_matches_host_input(orc, mtx):
     import torch
     pos, idx = _blas_case("rand5000")
