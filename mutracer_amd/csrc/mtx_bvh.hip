@@ -528,19 +528,24 @@ struct SmallBlockArrays {
   uint32_t ltmp[kSmall], X[kSmall], Z[kSmall], rk[kSmall];
   uint32_t kmin[3 * kMaxBins * 3], kmax[3 * kMaxBins * 3], cnt[3 * kMaxBins];
 };
-// Nodes of at most kRowNode primitives, with at most kRowNode bins, are split
-// four at a time, one to a row of 16 lanes: most nodes of a tree are that
-// small, the kernel is bound by vector instruction issue, and a wave with one
-// of them has work for a fifth of its lanes. 1M triangles in 8 bins: the
-// kernel takes 9.8 -> 4.1 ms, the build with its scene 19.1 -> 13.1 ms. (LDS
-// sized by the bins for a fourth workgroup per CU: 4.0 at the same three,
-// 4.1 at four, 16 registers spilled; twice the id atomics: the same time.)
+// Nodes of at most kRowNode primitives are split four at a time, one to a row
+// of 16 lanes: most nodes of a tree are that small, the kernel is bound by
+// vector instruction issue, and a wave with one of them has work for a
+// quarter of its lanes. Such a node fills at most kRowNode bins of an axis,
+// and only the filled ones are kept, numbered in order: an empty bin adds
+// nothing to a fold, and a split position behind one costs the same as the
+// filled position before it, which wins the tie.
+// 1M triangles, 8 bins: the kernel takes 9.8 -> 4.1 ms, the build with its
+// scene 18.2 -> 12.4 ms; 3M triangles, 32 bins: 24 ms a build, 41 with all
+// bins kept and four nodes to a wave up to 16 bins only. (LDS sized by the
+// bins for a fourth workgroup per CU: 4.0 ms at the same three, 4.1 at four,
+// 16 registers spilled; twice the id atomics: the same time.)
 constexpr int kRowNode = 16, kRows = 64 / kRowNode;
 // A wave's pending nodes hold two primitives or more each and are parts of
 // one queued node, beside at most kRows - 1 left of earlier ones.
 constexpr int kWaveStack = kWaveNode / 2 + kRows;
 struct SmallWaveArrays {
-  // one node's bins, or those of kRows nodes with at most kRowNode bins each
+  // one node's bins, or the filled ones of kRows nodes
   uint32_t kmin[3 * kMaxBins * 3], kmax[3 * kMaxBins * 3], cnt[3 * kMaxBins];
   uint32_t X[kWaveNode], Z[kWaveNode], tmp[kWaveNode];
   uint32_t stack[kWaveStack];  // pending node ids and their records: wide from the front, row nodes from the back
@@ -601,6 +606,14 @@ __device__ __forceinline__ uint32_t row_add(uint32_t v) {
   v += dpp_u<0x112, 0xf>(0u, v);
   v += dpp_u<0x114, 0xf>(0u, v);
   v += dpp_u<0x118, 0xf>(0u, v);
+  return v;
+}
+// The OR of a row's values, on all its lanes.
+__device__ __forceinline__ uint32_t row_or(uint32_t v) {
+  v |= dpp_u<0x128, 0xf>(0u, v);
+  v |= dpp_u<0x124, 0xf>(0u, v);
+  v |= dpp_u<0x122, 0xf>(0u, v);
+  v |= dpp_u<0x121, 0xf>(0u, v);
   return v;
 }
 // One step of a minimum over a row: the lower (cost, index) of this lane's and
@@ -715,32 +728,33 @@ __device__ __forceinline__ bool sah_split_wave(const uint32_t *kmin, const uint3
   return true;
 }
 
-// sah_split_wave for four nodes at once, one to a row of 16 lanes, bins <= 16:
-// lane b of the row holds bin b, the axes follow one another, and the scans,
-// the choice and the tie rules are the same within the row. `act` is the same
-// in a row; rows without a node run along. Returns whether the row's node
-// splits, the same on each of its lanes. Every lane of the wave calls it.
+// sah_split_wave for four nodes at once, one to a row of 16 lanes: lane b of
+// the row holds filled bin b of the axis (filled[axis] of them, at
+// kmin/kmax[(axis*stride + b)*3 + k] and cnt[axis*stride + b]), the axes
+// follow one another, and the scans, the choice and the tie rules are the same
+// within the row; out.pos is the number of a filled bin. `act` is the same in
+// a row; rows without a node run along. Returns whether the row's node splits,
+// the same on each of its lanes. Every lane of the wave calls it.
 __device__ __forceinline__ bool sah_split_row(const uint32_t *kmin, const uint32_t *kmax, const uint32_t *cnt,
-                                              int32_t bins, const NodeFrame &f, const double *minDim,
-                                              uint32_t nodePrims, bool act, Split &out) {
+                                              int32_t stride, const int32_t (&filled)[3], const NodeFrame &f,
+                                              const double *minDim, uint32_t nodePrims, bool act, Split &out) {
   const int lane = threadIdx.x & 63, b = lane & (kRowNode - 1), row0 = lane - b;
-  const bool isBin = b < bins;
-  const int src = row0 + (b < bins - 1 ? bins - 2 - b : 0);
   double bestCost = INFINITY;
   int bestIdx = 0x7fffffff;
 #pragma unroll
   for (int axis = 0; axis < 3; axis++) {
     const bool ok = act && f.extent[axis] > minDim[axis];
     if (!__any(ok)) continue;
-    const bool inb = ok && isBin;
-    const int fb = axis * bins + (isBin ? b : 0), rb = axis * bins + (isBin ? bins - 1 - b : 0);
+    const int m = filled[axis], src = row0 + (b < m - 1 ? m - 2 - b : 0);
+    const bool inb = ok && b < m;
+    const int fb = axis * stride + (inb ? b : 0), rb = axis * stride + (inb ? m - 1 - b : 0);
     const uint32_t cf = inb ? cnt[fb] : 0u, cr = inb ? cnt[rb] : 0u;
     float lmn[3], lmx[3], rmn[3], rmx[3];
     for (int k = 0; k < 3; k++) {
-      lmn[k] = cf ? unkey(kmin[fb * 3 + k]) : INFINITY;
-      lmx[k] = cf ? unkey(kmax[fb * 3 + k]) : -INFINITY;
-      rmn[k] = cr ? unkey(kmin[rb * 3 + k]) : INFINITY;
-      rmx[k] = cr ? unkey(kmax[rb * 3 + k]) : -INFINITY;
+      lmn[k] = inb ? unkey(kmin[fb * 3 + k]) : INFINITY;
+      lmx[k] = inb ? unkey(kmax[fb * 3 + k]) : -INFINITY;
+      rmn[k] = inb ? unkey(kmin[rb * 3 + k]) : INFINITY;
+      rmx[k] = inb ? unkey(kmax[rb * 3 + k]) : -INFINITY;
     }
     const uint32_t lc = row_add(cf), rcr = row_add(cr);
     for (int k = 0; k < 3; k++) {
@@ -752,7 +766,7 @@ __device__ __forceinline__ bool sah_split_row(const uint32_t *kmin, const uint32
     const uint32_t rightN = __shfl(rcr, src);
     float sr[6];
     for (int k = 0; k < 3; k++) { sr[k] = __shfl(rmn[k], src); sr[3 + k] = __shfl(rmx[k], src); }
-    if (ok && b < bins - 1) {
+    if (ok && b < m - 1) {
       double L[6], R[6];
       for (int k = 0; k < 3; k++) {
         L[k] = (double)lmn[k] < kFar ? (double)lmn[k] : kFar;
@@ -777,11 +791,12 @@ __device__ __forceinline__ bool sah_split_row(const uint32_t *kmin, const uint32
   out.axis = split ? bestIdx >> 6 : 0;
   out.pos = split ? bestIdx & 63 : 0;
   const float farF = (float)kFar;
-  const int bb = out.axis * bins + (isBin ? b : 0);
-  const bool filled = split && isBin && cnt[bb] != 0;
+  const int m = out.axis == 0 ? filled[0] : (out.axis == 1 ? filled[1] : filled[2]);
+  const bool inb = split && b < m;
+  const int bb = out.axis * stride + (inb ? b : 0);
   for (int sd = 0; sd < 2; sd++) {
-    const bool mine = filled && (sd == 0 ? b <= out.pos : b > out.pos);
-    const int at = row0 + (sd == 0 ? out.pos : bins - 1);
+    const bool mine = inb && (sd == 0 ? b <= out.pos : b > out.pos);
+    const int at = row0 + (sd == 0 ? out.pos : max(m - 1, 0));
     for (int k = 0; k < 3; k++) {
       const float vmn = __shfl(row_minmax<false>(mine ? unkey(kmin[bb * 3 + k]) : INFINITY), at);
       const float vmx = __shfl(row_minmax<true>(mine ? unkey(kmax[bb * 3 + k]) : -INFINITY), at);
@@ -978,19 +993,19 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
     }
   }
   // Phase 2: each wave takes queued nodes and splits them and their
-  // descendants on its own: nodes above rowNode primitives one at a time, then
+  // descendants on its own: nodes above kRowNode primitives one at a time, then
   // the others four at a time; a wave with fewer than four of these and no
   // wider node takes the next queued one first.
   __syncthreads();
   __threadfence_block();
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   SmallWaveArrays &W = sh.w[wv];
-  const uint32_t rowNode = bins <= kRowNode ? (uint32_t)kRowNode : 0u;
+  const int stride = min(bins, kRowNode);  // bins kept per axis of a row node
   const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
   int wide = 0, small = 0;  // pending nodes of each kind
   bool more = true;
   // A node's place among the pending ones; a single primitive stays a leaf.
-  auto place = [&](uint32_t n) -> int { return n > rowNode ? wide++ : kWaveStack - 1 - small++; };
+  auto place = [&](uint32_t n) -> int { return n > (uint32_t)kRowNode ? wide++ : kWaveStack - 1 - small++; };
   while (true) {
     if (more && wide == 0 && small < kRows) {
       uint32_t item = 0;
@@ -1077,36 +1092,43 @@ __global__ void __launch_bounds__(kBuildThreads) k_small_build(const SmallTask *
     const uint32_t n = valid ? nd.primCount : 0u, first = nd.leftFirst - base;
     const NodeFrame f = node_frame(nd.lo, nd.hi, bins, minDim);
     const bool act = valid && !(f.area == 0.0);
-    for (int i = lane; i < kRows * 3 * bins * 3; i += 64) { W.kmin[i] = 0xffffffffu; W.kmax[i] = 0u; }
-    for (int i = lane; i < kRows * 3 * bins; i += 64) W.cnt[i] = 0;
+    for (int i = lane; i < kRows * 9 * stride; i += 64) { W.kmin[i] = 0xffffffffu; W.kmax[i] = 0u; }
+    for (int i = lane; i < kRows * 3 * stride; i += 64) W.cnt[i] = 0;
     wave_sync();
-    uint32_t *const rmin = W.kmin + row * 9 * bins, *const rmax = W.kmax + row * 9 * bins,
-                    *const rcnt = W.cnt + row * 3 * bins;
+    uint32_t *const rmin = W.kmin + row * 9 * stride, *const rmax = W.kmax + row * 9 * stride,
+                    *const rcnt = W.cnt + row * 3 * stride;
     const bool live = act && (uint32_t)b < n;
-    const uint32_t p = live ? lp[first + b] : 0u;
-    float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    uint32_t p = 0;
+    float4 c = make_float4(0.0f, 0.0f, 0.0f, 0.0f), lo = c, hi = c;
     if (live) {
+      p = lp[first + b];
       c = cen[p];
-      const float4 lo = plo[p], hi = phi[p];
-      const float cc[3] = {c.x, c.y, c.z}, mn[3] = {lo.x, lo.y, lo.z}, mx[3] = {hi.x, hi.y, hi.z};
-      for (int ax = 0; ax < 3; ax++) {
-        const int bin = ax * bins + bin_of(cc[ax], f.nMin[ax], f.scale[ax], bins);
-        atomicAdd(&rcnt[bin], 1u);
+      lo = plo[p];
+      hi = phi[p];
+    }
+    const float cc[3] = {c.x, c.y, c.z}, mn[3] = {lo.x, lo.y, lo.z}, mx[3] = {hi.x, hi.y, hi.z};
+    int32_t mine[3], filled[3];
+#pragma unroll
+    for (int ax = 0; ax < 3; ax++) {
+      const int32_t bin = bin_of(cc[ax], f.nMin[ax], f.scale[ax], bins);
+      const uint32_t bit = live ? 1u << (bin & 31) : 0u, under = (1u << (bin & 31)) - 1u;
+      const uint32_t m0 = row_or(bin < 32 ? bit : 0u), m1 = bins > 32 ? row_or(bin < 32 ? 0u : bit) : 0u;
+      filled[ax] = __popc(m0) + __popc(m1);
+      mine[ax] = bin < 32 ? __popc(m0 & under) : __popc(m0) + __popc(m1 & under);
+      if (live) {
+        const int at = ax * stride + mine[ax];
+        atomicAdd(&rcnt[at], 1u);
         for (int k = 0; k < 3; k++) {
-          atomicMin(&rmin[bin * 3 + k], fkey(mn[k]));
-          atomicMax(&rmax[bin * 3 + k], fkey(mx[k]));
+          atomicMin(&rmin[at * 3 + k], fkey(mn[k]));
+          atomicMax(&rmax[at * 3 + k], fkey(mx[k]));
         }
       }
     }
     wave_sync();
     Split sp2;
-    const bool cuts = sah_split_row(rmin, rmax, rcnt, bins, f, minDim, n, act, sp2);
+    const bool cuts = sah_split_row(rmin, rmax, rcnt, stride, filled, f, minDim, n, act, sp2);
     const bool moves = cuts && live;
-    bool r = false;
-    if (moves) {
-      const float val = sp2.axis == 0 ? c.x : (sp2.axis == 1 ? c.y : c.z);
-      r = bin_of(val, pick3(f.nMin, sp2.axis), pick3(f.scale, sp2.axis), bins) > sp2.pos;
-    }
+    const bool r = moves && (sp2.axis == 0 ? mine[0] : (sp2.axis == 1 ? mine[1] : mine[2])) > sp2.pos;
     const uint32_t rmask = (uint32_t)(__ballot(r) >> row0) & 0xffffu;
     const uint32_t ex = (uint32_t)__popc(rmask & ((1u << b) - 1u)), nR = (uint32_t)__popc(rmask), nL = n - nR;
     uint32_t *const rX = W.X + row0, *const rZ = W.Z + row0;

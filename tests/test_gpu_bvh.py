@@ -63,13 +63,13 @@ def test_blas_bit_exact(orc, mtx, case, bins):
     assert info["max_leaf"] == ref["max_leaf"]
 
 
-@pytest.mark.parametrize("bins", [2, 8, 15, 16, 17])
+@pytest.mark.parametrize("bins", [2, 8, 16, 17, 32, 33, 64])
 @pytest.mark.parametrize("n", [2, 3, 15, 16, 17, 33, 63, 64, 65, 130, 1023, 1024, 1025, 1100])
 def test_blas_small_nodes_bit_exact(orc, mtx, n, bins):
     """Trees around the sizes where a node changes hands: 16 primitives (four
-    nodes to a wave, up to 16 bins), 64 (a node to a wave), 1024 (a subtree to
-    a workgroup). Half of the triangles lie on a line of shared centres, two
-    thirds of these at one point with zeros of both signs, so that ties,
+    nodes to a wave, filled bins only), 64 (a node to a wave), 1024 (a subtree to
+    a workgroup). Half of the triangles are flat and on a line, a third of
+    these at one point with zeros of both signs, so that ties,
     axes without extent and leaves of several primitives occur at every
     level."""
     rng = np.random.default_rng(n * 31 + bins)
