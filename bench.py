@@ -48,7 +48,7 @@ RAY_B = 32 + 32     # wavefront closest-hit query: ray in (origin, direction), h
 SAMPLE_B = 13 * 16 + 8  # per sample: read+write of 13 FP64 accumulator planes + the u32 count
 
 
-KERNEL_NAMES = {"wavefront": "k_wf_trace (closest-hit traversal of the wavefront sequence)",
+KERNEL_NAMES = {"wavefront": "k_wf_query (closest-hit traversal of the wavefront sequence)",
                 "megakernel": "k_render (megakernel)"}
 
 
@@ -349,8 +349,8 @@ def alpha_benchmark(opaque_sums, steps=3):
     """Cost of mask coverage at the headline workload: every material of the
     instanced field as a mask material whose coverage (opacity 1, cutoff
     0.5) covers everywhere. The image must equal the opaque render bit for
-    bit; the difference in time is what the coverage-testing shadow, walker
-    and tail kernels and the per-hit coverage resolution cost."""
+    bit; the difference in time is what the coverage-testing shadow rays and
+    tail kernel and the per-hit coverage resolution cost."""
     import torch
     from mutracer_amd import render, scene
     sc = scene.instanced_field()
@@ -463,7 +463,7 @@ def main():
     log(f"instrumented launch: {work}, rays {rays}")
     samples = WIDTH * HEIGHT * SPP
     if args.kernel == "wavefront":
-        # Dominant kernel: the closest-hit trace k_wf_trace (ray in + hit out +
+        # Dominant kernel: the closest hits of k_wf_query (ray in + hit out +
         # node/triangle/instance fetches), counted over its own launches only
         # (the tail kernel's traversal work is the "tail" group).
         wf = work["wavefront"]
@@ -535,7 +535,7 @@ def main():
         serving = serving_benchmark(n_jobs=args.serving_jobs, per_sample=args.serving_per_sample)
 
     traffic = profile_value("wf_trace_c2_1080p_traffic.txt", "traffic_bytes_per_step")
-    valu = profile_value("wf_c2_1080p_valu_issue.txt", "k_wf_trace_valu_issue_frac")
+    valu = profile_value("wf_c2_1080p_valu_issue.txt", "k_wf_query_closest_valu_issue_frac")
     out = {
         "metric": METRIC, "value": round(value, 3), "unit": "Msamples/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": round(ms_per_step, 3), "higher_is_better": True, "scaling": "weak",
@@ -553,9 +553,10 @@ def main():
                      "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": traffic, "kernel": KERNEL_NAMES[args.kernel], "kernel_ms": round(kernel_ms, 3),
                      "algorithmic_bytes_per_step": int(alg_bytes),
-                     # The roof that binds this kernel is vector instruction issue, not HBM: the
-                     # algorithmic bytes mostly hit in L2; measured traffic and issue rate follow.
-                     "binding_roof": "valu_issue",
+                     # The roof that binds this kernel is the load units' address rate (78% busy), then
+                     # vector instruction issue, not HBM: the algorithmic bytes mostly hit in L2;
+                     # measured traffic and issue rate follow.
+                     "binding_roof": "vector_load_address_rate",
                      "valu_issue_frac": valu,
                      "hbm_traffic_frac": (round(traffic / (kernel_ms / 1e3) / 1e9 / HBM_PEAK_GBS, 4)
                                           if traffic else None),

@@ -5,13 +5,14 @@
 // high-occupancy kernels and shading in its own kernel:
 //
 //   generate  camera rays for every path of the generation
-//   per event e = 0 .. min(3 * bounces, 50):
-//     trace   closest hit for the paths in queue e          (LDS short stack)
+//   per event e = 0 .. event_limit():
+//     query   closest hits for the paths in queue e and, in the same launch,
+//             any-hit for the shadow queue of event e - 1, adding the payload
+//             of each unoccluded ray to its path's radiance
 //     shade   shade_event(): emission, NEE candidate choice, BSDF sample,
 //             Russian roulette; appends the path to queue e+1 when it
 //             continues and its shadow ray to the shadow queue of event e
-//     shadow  any-hit for the shadow queue; adds the payload of each
-//             unoccluded ray to its path's radiance
+//   query     the last event's shadow queue
 //   accumulate each pixel's samples, in sample order, into the FP64 running
 //             sums and advance the per-pixel sample counter
 //
