@@ -153,7 +153,11 @@ typedef struct mtx_hit {
 
 /* querySceneSoftware (intersect.wgsl.ts:660-684): closest hit for `count`
  * device-resident rays into device-resident hits on `stream` (hipStream_t,
- * NULL = default). Asynchronous; synchronize the stream before reading. */
+ * NULL = default). Asynchronous; synchronize the stream before reading.
+ * Queries of several threads on one stream follow one another. A closest-hit
+ * or counting query recorded into a graph uses its stream's work counters on
+ * every replay: no query on that stream and no graph recorded on it may run
+ * beside the replay (mtx_trace_any has no counters there). */
 int32_t mtx_trace_closest(mtx_handle accel, const mtx_ray *rays, uint32_t count, mtx_hit *hits,
                           uint32_t flags, void *stream);
 

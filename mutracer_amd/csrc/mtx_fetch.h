@@ -39,6 +39,10 @@ constexpr uint32_t kCtrStride = 128;
 // With the counters on one line, an atomic per 64 rays and eight more for
 // every wave's end, the 1.6M closest-hit rays of a 256 x 256 x 8 Cornell
 // generation took 2.27 ms; with this queue and trace_queue 0.62 ms.
+//
+// kStatic: no counters. The waves share the chunks out among themselves, wave
+// w taking w, w + waves, ... , so calls that overlap on a stream share nothing.
+template <bool kStatic>
 struct WorkQueue {
   uint32_t n, chunk, chunks;
   uint32_t *ctr;
@@ -73,12 +77,23 @@ struct WorkQueue {
     const uint32_t c = seg_lo(seg) + (reverse ? seg_waves(seg) - 1u - rank : rank);
     base = limit = 0;
     open = true;
+    if (kStatic) {
+      seg = blockIdx.x * (blockDim.x >> 6) + wave;
+      if (seg < chunks) set(seg);
+      return;
+    }
     if (c < seg_lo(seg + 1u)) set(c);
   }
 
   // Entries left for this wave (fetches a chunk when the current one is used up).
   __device__ __forceinline__ bool more() {
     if (base < limit) return true;
+    if (kStatic) {
+      const uint32_t waves = gridDim.x * (blockDim.x >> 6);
+      if (seg >= chunks || chunks - seg <= waves) return false;
+      seg += waves;
+      return set(seg);
+    }
     while (open) {
       uint32_t first = seg_lo(seg) + seg_waves(seg), end = seg_lo(seg + 1u);
       if (first < end) {

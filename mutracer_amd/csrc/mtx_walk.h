@@ -45,14 +45,14 @@ struct RayIn {
 // a closest-hit query (the last one given is the closest), covers(id, slot,
 // tri, barycentrics) is the coverage test of masked instances (any hit), and
 // done(id, any, counters) ends the entry. `ctr` is the queue's chunk counters
-// and kReverse its order of waves (WorkQueue).
-template <bool kAnyHit, bool kCount, bool kMulti, bool kMasked, bool kReverse, class Stack, class Load, class Hit, class Covers, class Done>
+// (none with kStatic) and kReverse its order of waves (WorkQueue).
+template <bool kAnyHit, bool kCount, bool kMulti, bool kMasked, bool kReverse, bool kStatic, class Stack, class Load, class Hit, class Covers, class Done>
 __device__ __forceinline__ void trace_queue(uint32_t n, uint32_t *ctr, const AccelView &one, bool doubleSided, Stack &st,
                                             Load &&load, Hit &&hit, Covers &&covers, Done &&done) {
   // cur >= 0: the interior node to visit; cur < kIdle: a leaf (of the BLAS
   // while inBlas, else of the TLAS); kReturn: the current subtree is done.
   constexpr int32_t kReturn = -1, kIdle = -2;
-  WorkQueue wq(n, ctr, kReverse);
+  WorkQueue<kStatic> wq(n, ctr, kReverse);
   const uint32_t lane = lane_id();
   uint32_t id = 0;
   f3 ro = splat(0.0f), rd = ro, winv = ro, o = ro, invD = ro, shear = ro;

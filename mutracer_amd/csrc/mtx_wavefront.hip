@@ -361,7 +361,7 @@ __device__ __forceinline__ void closest_hits(const WfLaunch &L, const WfBuffers 
       hits += any ? 1u : 0u;
     }
   };
-  trace_queue<false, kCount, kMulti, false, false>(n, W.counts + kWfXcdBase + 2 * event, one, event != 0, st, load,
+  trace_queue<false, kCount, kMulti, false, false, false>(n, W.counts + kWfXcdBase + 2 * event, one, event != 0, st, load,
                                                    hit, covers, done);
   if (kCount) {
     const uint64_t v[5] = {(blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u, boxes, tris, instances, hits};
@@ -404,7 +404,7 @@ __device__ __forceinline__ void shadow_rays(const WfLaunch &L, const WfBuffers &
       instances += c.instances;
     }
   };
-  trace_queue<true, kCount, kMulti, kAlpha, true>(n, W.counts + kWfXcdBase + 2 * event + 1, one, true, st, load, hit,
+  trace_queue<true, kCount, kMulti, kAlpha, true, false>(n, W.counts + kWfXcdBase + 2 * event + 1, one, true, st, load, hit,
                                                   covers, done);
   if (kCount) {
     const uint64_t v[4] = {boxes, tris, instances, (blockIdx.x == 0 && threadIdx.x == 0) ? (uint64_t)n : 0u};

@@ -182,3 +182,96 @@ def test_query_sizes_bit_exact(orc, env, queue_scene, n):
     torch.cuda.synchronize()
     o = o.cpu().numpy()
     assert np.array_equal(o[:n].astype(np.uint32), occ[:n]) and o[n] == 7
+
+
+def test_any_hit_threads_on_one_stream(orc, env, queue_scene):
+    """Occlusion queries of two threads on the default stream, with more rays
+    than the waves start with: every query answers all of its rays."""
+    import threading
+    torch, accel, W = env
+    scene, acc, rays, ref, occ = queue_scene
+    reps, bad = 60, []
+    dev = [torch.from_numpy(np.tile(rays[k::2], (4, 1))).cuda() for k in range(2)]
+    exp = [torch.from_numpy(np.tile(occ[k::2].astype(np.int32), 4)).cuda() for k in range(2)]
+    outs = [torch.full((reps, d.shape[0]), 7, dtype=torch.int32, device="cuda") for d in dev]
+    torch.cuda.synchronize()
+
+    def ask(k):
+        try:
+            for i in range(reps):
+                acc.trace_any(dev[k], outs[k][i])
+        except Exception as e:
+            bad.append(e)
+
+    threads = [threading.Thread(target=ask, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not bad
+    for k in range(2):
+        assert bool((outs[k] == exp[k]).all())
+
+
+# The waves' first chunks only, and a second chunk for some of them.
+@pytest.mark.parametrize("n", [1, 6145, 393_217, 400_000])
+def test_any_hit_recorded(orc, env, queue_scene, n):
+    """An occlusion query recorded into a graph, replayed between eager work."""
+    torch, accel, W = env
+    scene, acc, rays, ref, occ = queue_scene
+    r = torch.from_numpy(rays[:n]).cuda()
+    o = torch.full((n + 1,), 7, dtype=torch.int32, device="cuda")
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        acc.trace_any(r, o, stream=s)  # the stream's scratch
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        acc.trace_any(r, o, stream=s)
+    for _ in range(3):
+        o.fill_(7)
+        g.replay()
+        acc.trace_any(r[:1], o[:1])
+        torch.cuda.synchronize()
+        got = o.cpu().numpy()
+        assert np.array_equal(got[:n].astype(np.uint32), occ[:n]) and got[n] == 7
+
+
+def test_any_hit_graphs_side_by_side(orc, env):
+    """Two occlusion queries recorded on one stream, replayed on two at once.
+    (A scene whose stacks fit in LDS: spilled ones belong to a stream.)"""
+    torch, accel, W = env
+    pos, idx = W.sphere_mesh(20, 10)
+    scene = orc.assemble_scene([dict(positions=pos, indices=idx)],
+                               dict(mesh=[0], transform=[W.identity_transform()], material=[0]))
+    blas = accel.Blas(pos, idx)
+    assert blas.info()["max_depth"] < 16
+    acc = accel.Accel([blas], [0], [W.identity_transform()])
+    rng = np.random.default_rng(5)
+    rays = np.zeros((50_000, 8), np.float32)
+    rays[:, 0:3], rays[:, 4:7] = rng.uniform(-1.5, 1.5, (50_000, 3)), rng.normal(size=(50_000, 3))
+    rays[:, 3] = rng.uniform(0.0, 2.0, 50_000)
+    occ = scene.any(rays).astype(np.int32)
+    rec, streams, work = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()], []
+    for k in range(2):
+        r = torch.from_numpy(np.tile(rays[k::2], (40, 1))).cuda()
+        e = torch.from_numpy(np.tile(occ[k::2], 40)).cuda()
+        o = torch.full((r.shape[0],), 7, dtype=torch.int32, device="cuda")
+        acc.trace_any(r, o, stream=rec)
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=rec):
+            acc.trace_any(r, o, stream=rec)
+        work.append((g, r, o, e))
+    for _ in range(5):
+        for g, r, o, e in work:
+            o.fill_(7)
+        torch.cuda.synchronize()
+        for _ in range(4):
+            for s, (g, r, o, e) in zip(streams, work):
+                with torch.cuda.stream(s):
+                    g.replay()
+        torch.cuda.synchronize()
+        for g, r, o, e in work:
+            assert bool((o == e).all())
