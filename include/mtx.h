@@ -154,7 +154,9 @@ typedef struct mtx_hit {
 /* querySceneSoftware (intersect.wgsl.ts:660-684): closest hit for `count`
  * device-resident rays into device-resident hits on `stream` (hipStream_t,
  * NULL = default). Asynchronous; synchronize the stream before reading.
- * Queries of several threads on one stream follow one another. A closest-hit
+ * The library keeps the traversal stacks' spill memory of every stream it was
+ * called on: 576 bytes per ray of its largest query (rounded up to the grid's
+ * waves), at most about 270 MB. Queries of several threads on one stream follow one another. A closest-hit
  * or counting query recorded into a graph uses its stream's work counters on
  * every replay: no query on that stream and no graph recorded on it may run
  * beside the replay (mtx_trace_any has no counters there). */

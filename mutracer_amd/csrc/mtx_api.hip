@@ -42,8 +42,12 @@ k_trace(const AccelView *__restrict__ viewp, const mtx_ray *__restrict__ rays, u
   constexpr bool kAny = kMode == 1 || kMode == 4;
   __shared__ int32_t lds[kMinLdsStack * kTraceBlock];
   const AccelView acc = *viewp;
-  LaneStackT<kMinLdsStack> st{lds + threadIdx.x, kTraceBlock,
-                              spill + ((size_t)blockIdx.x * kTraceBlock + threadIdx.x) * (kMaxStack - kMinLdsStack)};
+  // Only the lanes that take rays have a spill slice.
+  const uint32_t wave = blockIdx.x * (kTraceBlock / 64) + (threadIdx.x >> 6);
+  const uint32_t lanes = queue_lanes(n, gridDim.x * (kTraceBlock / 64));
+  LaneStackT<kMinLdsStack> st{
+      lds + threadIdx.x, kTraceBlock,
+      spill + ((size_t)wave * lanes + min(lane_id(), lanes - 1u)) * (kMaxStack - kMinLdsStack)};
   const bool doubleSided = kAny || (flags & MTX_TRACE_DOUBLE_SIDED) != 0;
   auto load = [&](uint32_t i, RayIn &r) {
     const float4 *r4 = reinterpret_cast<const float4 *>(rays + i);
@@ -112,15 +116,15 @@ uint32_t trace_grid() {
 
 // Each lane owns kMaxStack - kLds entries at lane * (kMaxStack - kLds): sized
 // for the smallest LDS depth any kernel uses. The caller holds S.m.
-static int32_t *spill_of(StreamScratch &S, uint32_t blocksNeeded, uint32_t blockThreads) {
-  const size_t need = (size_t)blocksNeeded * blockThreads * (kMaxStack - kMinLdsStack);
+static int32_t *spill_of(StreamScratch &S, size_t lanes) {
+  const size_t need = lanes * (kMaxStack - kMinLdsStack);
   if (S.spill.count < need) S.spill = DevBuf<int32_t>(need);
   return S.spill.ptr;
 }
 int32_t *spill_for(hipStream_t s, uint32_t blocksNeeded, uint32_t blockThreads) {
   auto S = scratch_of(s);
   std::lock_guard<std::mutex> g(S->m);
-  return spill_of(*S, blocksNeeded, blockThreads);
+  return spill_of(*S, (size_t)blocksNeeded * blockThreads);
 }
 // Whether launches on s are being recorded into a graph.
 static bool recording(hipStream_t s) {
@@ -175,7 +179,8 @@ static void launch_trace(int mode, const Accel &A, const mtx_ray *rays, uint32_t
   if (mode == 1 && recording(s)) mode = 4;
   auto S = scratch_of(s);
   std::lock_guard<std::mutex> g(S->m);
-  int32_t *spill = spill_of(*S, grid, kTraceBlock);
+  const uint32_t waves = grid * (kTraceBlock / 64);
+  int32_t *spill = spill_of(*S, (size_t)waves * queue_lanes(n, waves));
   if (mode != 4 && !S->counters.ptr) S->counters.alloc(kXcds * kCtrStride);
   launch_query(mode, grid, A, rays, n, hits, out, flags, spill, S->counters.ptr, s);
 }

@@ -27,6 +27,12 @@ constexpr int kRefill = 16;
 // own, so that an atomic moves no line between XCDs.
 constexpr uint32_t kCtrStride = 128;
 
+// Lanes of a wave that take entries when `waves` waves share a queue of n.
+constexpr uint32_t queue_lanes(uint32_t n, uint32_t waves) {
+  const uint64_t per = ((uint64_t)n + waves - 1u) / waves;
+  return per < 1u ? 1u : (per > 64u ? 64u : (uint32_t)per);
+}
+
 // A wave's view of a queue of n entries that all waves of the grid empty
 // together. The queue is cut into chunks, the chunks into one contiguous
 // segment per XCD (block b runs on XCD b % 8), and every wave starts with a
@@ -65,8 +71,7 @@ struct WorkQueue {
   // second of two queues that one launch empties.
   __device__ __forceinline__ WorkQueue(uint32_t n_, uint32_t *ctr_, bool reverse) : n(n_), ctr(ctr_) {
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
-    const uint32_t per = (uint32_t)(((uint64_t)n + waves - 1u) / waves);
-    lanes = (int)min(64u, max(1u, per));
+    lanes = (int)queue_lanes(n, waves);
     chunk = lanes < 64 ? (uint32_t)lanes : 64u * min(4u, max(1u, n / (waves * 512u)));
     chunks = (n + chunk - 1u) / chunk;
     laneMask = lanes == 64 ? ~0ull : (1ull << lanes) - 1ull;

@@ -275,3 +275,25 @@ def test_any_hit_graphs_side_by_side(orc, env):
         torch.cuda.synchronize()
         for g, r, o, e in work:
             assert bool((o == e).all())
+
+
+# One ray a wave on part of the grid, on all of it, eight a wave.
+@pytest.mark.parametrize("n,mib", [(1000, 4), (4096, 8), (40_000, 40)])
+def test_spill_memory_of_short_queries(env, queue_scene, n, mib):
+    """A stream's first queries allocate stack memory for the rays they have
+    (576 bytes a ray), not for every lane of the grid."""
+    torch, accel, W = env
+    scene, acc, rays, ref, occ = queue_scene
+    r = torch.from_numpy(rays[:n]).cuda()
+    h = torch.zeros((n, 8), dtype=torch.int32, device="cuda")
+    o = torch.zeros((n,), dtype=torch.int32, device="cuda")
+    acc.trace_closest(r, h)  # the kernels' code is loaded
+    acc.trace_any(r, o)
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    acc.trace_closest(r, h, stream=s)
+    acc.trace_any(r, o, stream=s)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] <= mib << 20
+    assert np.array_equal(o.cpu().numpy().astype(np.uint32), occ[:n])
