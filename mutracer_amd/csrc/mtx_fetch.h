@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "mtx_split.h"
+
 namespace mtx {
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
@@ -26,12 +28,6 @@ constexpr int kRefill = 16;
 // Words between the chunk counters of two XCDs: each counter on lines of its
 // own, so that an atomic moves no line between XCDs.
 constexpr uint32_t kCtrStride = 128;
-
-// Lanes of a wave that take entries when `waves` waves share a queue of n.
-constexpr uint32_t queue_lanes(uint32_t n, uint32_t waves) {
-  const uint64_t per = ((uint64_t)n + waves - 1u) / waves;
-  return per < 1u ? 1u : (per > 64u ? 64u : (uint32_t)per);
-}
 
 // A wave's view of a queue of n entries that all waves of the grid empty
 // together. The queue is cut into chunks, the chunks into one contiguous
@@ -72,8 +68,8 @@ struct WorkQueue {
   __device__ __forceinline__ WorkQueue(uint32_t n_, uint32_t *ctr_, bool reverse) : n(n_), ctr(ctr_) {
     const uint32_t waves = gridDim.x * (blockDim.x >> 6);
     lanes = (int)queue_lanes(n, waves);
-    chunk = lanes < 64 ? (uint32_t)lanes : 64u * min(4u, max(1u, n / (waves * 512u)));
-    chunks = (n + chunk - 1u) / chunk;
+    chunk = queue_chunk(n, waves);
+    chunks = queue_chunks(n, chunk);
     laneMask = lanes == 64 ? ~0ull : (1ull << lanes) - 1ull;
     refillMin = min(lanes, kRefill);
     seg = blockIdx.x % (uint32_t)kXcds;
