@@ -33,6 +33,7 @@
 #include <mutex>
 #include <unordered_map>
 
+#include "mtx_fetch.h"
 #include "mtx_scene.h"
 
 namespace mtx {
@@ -516,13 +517,6 @@ struct SmallTask {
 // workgroup work on four such subtrees at once.
 constexpr int kWaveNode = 64;
 constexpr int kBuildWaves = kBuildThreads / 64;
-
-// Ordering point for LDS between the lanes of one wave.
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 struct SmallBlockArrays {
   uint32_t ltmp[kSmall], X[kSmall], Z[kSmall], rk[kSmall];

@@ -10,6 +10,15 @@ namespace mtx {
 
 __device__ __forceinline__ uint32_t lane_id() { return threadIdx.x & 63u; }
 
+// Ordering point for LDS between the lanes of one wave: what they stored
+// before it, the others load after it. (The barrier alone orders nothing in
+// memory, it only keeps the instructions together.)
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 constexpr int kXcds = 8;
 
 // Occupancy the register allocator must reach for the traversal kernels

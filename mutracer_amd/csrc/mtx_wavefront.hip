@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
       }
       at = n - at > nWaves * per ? at + nWaves * per : n;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     // The last 64 paths of a full class, or what the classes have left.
     uint32_t p = 0, taken = 0;
     bool active = false;
@@ -239,7 +239,7 @@ __global__ void __launch_bounds__(kWfShadeBlock, kWaves) k_wf_shade(const WfLaun
       cnt[c] -= k;
       taken += k;
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     if (taken == 0u) break;
     bool alive = false;
     ShadowReq sr;

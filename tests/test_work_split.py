@@ -41,3 +41,14 @@ def test_every_entry_in_one_chunk(program, waves):
         assert lanes == min(64, max(1, -(-n // waves)))
         assert chunk >= lanes and chunk <= 256
         assert (chunks - 1) * chunk < n <= chunks * chunk, (n, chunk, chunks)
+
+
+def test_wave_barriers_order_memory():
+    """The bare wave barrier orders no memory: lanes that hand values to one
+    another through LDS meet in wave_sync(), its only user."""
+    csrc, uses = os.path.join(ROOT, "mutracer_amd", "csrc"), []
+    for f in sorted(os.listdir(csrc)):
+        if f.endswith((".h", ".hip", ".cpp")):
+            text = open(os.path.join(csrc, f)).read()
+            uses += [f] * text.count("__builtin_amdgcn_wave_barrier(")
+    assert uses == ["mtx_fetch.h"]
