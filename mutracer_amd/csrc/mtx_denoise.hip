@@ -687,7 +687,8 @@ struct DenoiserObj {
   // Prefilters of the albedo and normal guides (clean-auxiliary models).
   std::shared_ptr<DenoiserObj> auxAlbedo, auxNormal;
   hipStream_t stream = nullptr;
-  hipStream_t copies[2] = {nullptr, nullptr};  // beside `stream` for large host copies, made by the first
+  HostBuf result;                              // on its way to the caller
+  hipStream_t copies[2] = {nullptr, nullptr};  // beside `stream` for large uploads, made by the first
   std::mutex busy;
   ~DenoiserObj() {
     for (hipStream_t c : copies)
@@ -925,49 +926,67 @@ static void download_layer(DenoiserObj &D, int i, int H, int W, float *out, hipS
     for (int c = 0; c < co; c++) out[p * co + c] = D.bf16 ? bf16_to_f32(h[p * cs + c]) : f16_to_f32(h[p * cs + c]);
 }
 
-// Three host <-> device copies, done when it returns. A copy of pageable
-// memory goes at the pace of the thread that issues it, so large ones take a
-// thread and a stream each (blocking streams, ordered after earlier
-// null-stream work as D.stream is). A 1080p run (100 MB in, 33 MB out) took
-// 13.9 ms; with the result straight into the caller's buffer 6.5, with the
-// uploads on threads 5.8, with the download too 4.8.
-struct HostCopy {
-  void *dst;
-  const void *src;
-  size_t bytes;
-  hipMemcpyKind kind;
-};
-constexpr size_t kThreadedCopyBytes = 4u << 20;  // 509 x 287 (7 MB in): 0.73 -> 0.64 ms; small runs need no threads
-static void host_copies(DenoiserObj &D, const HostCopy (&c)[3]) {
-  if (c[0].bytes + c[1].bytes + c[2].bytes < kThreadedCopyBytes) {
-    for (const HostCopy &k : c)
-      if (k.bytes) MTX_HIP(hipMemcpyAsync(k.dst, k.src, k.bytes, k.kind, D.stream));
-    MTX_HIP(hipStreamSynchronize(D.stream));
+// Host copies of a run. Its images come from and go to pageable memory, and a
+// copy of that goes at the pace of the thread that issues it, so large images
+// go up on three threads, each with a stream (blocking streams, ordered after
+// earlier null-stream work as D.stream is). The result passes through pinned
+// memory of the denoiser's own and is copied to the caller's buffer once it is
+// whole: a run that fails leaves the caller's buffer as it was (1080p 4.4 ms a
+// run with parts of the result straight into that buffer, 4.6 so).
+constexpr size_t kThreadedUploadBytes = 4u << 20;  // 509 x 287 (7 MB in): 0.73 -> 0.64 ms; small runs need no threads
+constexpr size_t kThreadedCopyBytes = 4u << 20;    // results that threads copy to the caller
+
+// work(0), work(1) and work(2), on threads of their own as far as there are any to be had.
+template <class Work>
+static void on_threads(const Work &work) {
+  std::thread t[2];
+  try {
+    for (int k = 0; k < 2; k++) t[k] = std::thread(work, k + 1);
+  } catch (const std::exception &) {
+  }
+  work(0);
+  for (int k = 0; k < 2; k++) {
+    if (t[k].joinable()) t[k].join();
+    else work(k + 1);
+  }
+}
+
+static void upload_images(DenoiserObj &D, const float *const (&src)[3], size_t bytes) {
+  bool threads = 3 * bytes >= kThreadedUploadBytes;
+  for (hipStream_t &s : D.copies) {
+    if (!threads || s) continue;
+    threads = hipStreamCreate(&s) == hipSuccess;
+    if (!threads) (void)hipGetLastError();
+  }
+  if (!threads) {
+    for (int k = 0; k < 3; k++)
+      MTX_HIP(hipMemcpyAsync(D.io[k].ptr, src[k], bytes, hipMemcpyHostToDevice, D.stream));
     return;
   }
   int dev = 0;
   MTX_HIP(hipGetDevice(&dev));
-  for (hipStream_t &s : D.copies)
-    if (!s) MTX_HIP(hipStreamCreate(&s));
   hipError_t err[3] = {hipSuccess, hipSuccess, hipSuccess};
-  auto copy = [&](int k) {
-    if (!c[k].bytes) return;
-    const hipStream_t st = k ? D.copies[k - 1] : D.stream;
+  on_threads([&](int k) {
+    const hipStream_t s = k ? D.copies[k - 1] : D.stream;
     err[k] = hipSetDevice(dev);
-    if (err[k] == hipSuccess) err[k] = hipMemcpyAsync(c[k].dst, c[k].src, c[k].bytes, c[k].kind, st);
-    if (err[k] == hipSuccess) err[k] = hipStreamSynchronize(st);
-  };
-  std::thread t[2];
-  try {
-    for (int k = 0; k < 2; k++) t[k] = std::thread(copy, k + 1);
-  } catch (const std::exception &) {  // no thread to be had: the remaining copies run here
-  }
-  copy(0);
-  for (int k = 0; k < 2; k++) {
-    if (t[k].joinable()) t[k].join();
-    else copy(k + 1);
-  }
+    if (err[k] == hipSuccess) err[k] = hipMemcpyAsync(D.io[k].ptr, src[k], bytes, hipMemcpyHostToDevice, s);
+    if (err[k] == hipSuccess) err[k] = hipStreamSynchronize(s);
+  });
   for (hipError_t e : err) MTX_HIP(e);
+}
+
+static void download_result(DenoiserObj &D, float *out, size_t bytes) {
+  char *const from = static_cast<char *>(D.result.ensure(bytes, true));
+  MTX_HIP(hipMemcpyAsync(from, D.io[3].ptr, bytes, hipMemcpyDeviceToHost, D.stream));
+  MTX_HIP(hipStreamSynchronize(D.stream));
+  if (bytes < kThreadedCopyBytes) {
+    std::memcpy(out, from, bytes);
+    return;
+  }
+  const size_t part = bytes / 3;
+  on_threads([&](int k) {
+    std::memcpy(reinterpret_cast<char *>(out) + k * part, from + k * part, k == 2 ? bytes - 2 * part : part);
+  });
 }
 
 // One image through a network, tile by tile: tiles of max_tile pixels (0 =
@@ -1194,9 +1213,7 @@ int32_t mtx_denoiser_run(mtx_handle handle, uint32_t width, uint32_t height, con
     }
     hipStream_t s = D->stream;
     const size_t bytes = n * sizeof(float4);
-    host_copies(*D, {{D->io[0].ptr, color, bytes, hipMemcpyHostToDevice},
-                     {D->io[1].ptr, albedo, bytes, hipMemcpyHostToDevice},
-                     {D->io[2].ptr, normal, bytes, hipMemcpyHostToDevice}});
+    upload_images(*D, {color, albedo, normal}, bytes);
     const float4 *guideA = D->io[1].ptr, *guideN = D->io[2].ptr;
     if (D->auxAlbedo) {
       // Clean auxiliary guides (WGPURenderingPipeline.ts:1352-1440,
@@ -1211,13 +1228,7 @@ int32_t mtx_denoiser_run(mtx_handle handle, uint32_t width, uint32_t height, con
     denoise_image(*D, D->maxTile, D->overlap, D->io[0].ptr, guideA, guideN, (int)width, (int)height, kNetBeauty,
                   D->io[3].ptr, s);
     MTX_HIP(hipGetLastError());
-    MTX_HIP(hipStreamSynchronize(s));  // the caller's buffer is written only after the run has succeeded
-    const size_t part = n / 3;
-    float4 *out = reinterpret_cast<float4 *>(output);
-    host_copies(*D, {{out, D->io[3].ptr, part * sizeof(float4), hipMemcpyDeviceToHost},
-                     {out + part, D->io[3].ptr + part, part * sizeof(float4), hipMemcpyDeviceToHost},
-                     {out + 2 * part, D->io[3].ptr + 2 * part, (n - 2 * part) * sizeof(float4),
-                      hipMemcpyDeviceToHost}});
+    download_result(*D, output, bytes);
     return MTX_OK;
   } catch (const Error &e) {
     set_error(err, cap, e.what());

@@ -3,7 +3,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <cstdio>
+#include <cstdlib>
 #include <cstring>
+#include <new>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -76,6 +78,37 @@ struct DevBuf {
     download(v.data(), n, s);
     MTX_HIP(hipStreamSynchronize(s));
     return v;
+  }
+};
+
+// Owning host memory, pinned if asked for and to be had.
+struct HostBuf {
+  void *ptr = nullptr;
+  size_t bytes = 0;
+  bool pinned = false;
+  HostBuf() = default;
+  HostBuf(const HostBuf &) = delete;
+  HostBuf &operator=(const HostBuf &) = delete;
+  ~HostBuf() { release(); }
+  // At least n bytes; what it held before is lost if it has to grow or change.
+  void *ensure(size_t n, bool pin) {
+    if (bytes >= n && (pinned || !pin)) return ptr;
+    release();
+    if (pin) {
+      pinned = hipHostMalloc(&ptr, n, 0) == hipSuccess;
+      if (!pinned) (void)hipGetLastError();
+    }
+    if (!pinned) ptr = std::malloc(n);
+    if (!ptr) throw std::bad_alloc();
+    bytes = n;
+    return ptr;
+  }
+  void release() {
+    if (pinned) (void)hipHostFree(ptr);
+    else std::free(ptr);
+    ptr = nullptr;
+    bytes = 0;
+    pinned = false;
   }
 };
 

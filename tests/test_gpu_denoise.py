@@ -316,6 +316,78 @@ def test_run_host_copies(net, h, w):
         assert np.array_equal(out[..., 3], images[0][..., 3])
 
 
+# A hipMemcpyAsync that can be told to refuse one copy from the device.
+REFUSE = """
+#include <stddef.h>
+#include <dlfcn.h>
+typedef int (*copy_fn)(void *, const void *, size_t, int, void *);
+static copy_fn next;
+static int left;
+int refuse_from(const char *runtime) {
+  void *h = dlopen(runtime, RTLD_NOW | RTLD_NOLOAD);
+  next = h ? (copy_fn)dlsym(h, "hipMemcpyAsync") : 0;
+  return next != 0;
+}
+void refuse(int nth) { left = nth; }
+int refused(void) { return left == 0; }
+int hipMemcpyAsync(void *dst, const void *src, size_t n, int kind, void *stream) {
+  if (kind == 2 && left > 0 && --left == 0) return 999;
+  return next(dst, src, n, kind, stream);
+}
+"""
+FAILED_RUNS = """
+import ctypes as C, sys
+lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before the runtime: the library's calls go through it
+import numpy as np
+from mutracer_amd import abi, denoise
+abi.lib()
+runtime = {l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l}
+assert len(runtime) == 1 and lib.refuse_from(runtime.pop().encode())
+h, w = int(sys.argv[2]), int(sys.argv[3])
+rng = np.random.default_rng(3)
+im = [rng.random((h, w, 4), np.float32) for _ in range(3)]
+d = denoise.Denoiser("fp16")
+want = d.run(*im)
+P = lambda a: a.ctypes.data_as(C.c_void_p)
+failures = 0
+for run in range(12):
+    for nth in range(1, 5):
+        out = np.full((h, w, 4), -7.0, np.float32)
+        lib.refuse(nth)
+        err = abi.errbuf()
+        code = abi.lib().mtx_denoiser_run(d.handle.value, w, h, P(im[0]), P(im[1]), P(im[2]), P(out), out.size, err, 512)
+        if lib.refused():
+            assert code != abi.MTX_OK, (run, nth)
+            assert (out == -7.0).all(), (run, nth, "a failed run wrote to the output")
+            failures += 1
+        else:
+            assert code == abi.MTX_OK and np.array_equal(out, want), (run, nth)
+            break
+    lib.refuse(0)
+assert failures >= 12
+print("PASS")
+"""
+
+
+@pytest.mark.parametrize("h,w", [(64, 80), (287, 509), (819, 854)])
+def test_failed_download_leaves_the_output(net, tmp_path, h, w):
+    """A run whose copy of the result from the device is refused (by a
+    stand-in for the runtime's copy call, in a process of its own) fails and
+    leaves the caller's buffer as it was, in first and in later runs; the
+    runs after it give the result."""
+    import subprocess
+    import sys
+    (tmp_path / "refuse.c").write_text(REFUSE)
+    (tmp_path / "runs.py").write_text(FAILED_RUNS)
+    so = tmp_path / "refuse.so"
+    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", str(tmp_path / "refuse.c"), "-o", str(so), "-ldl"],
+                   check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, str(tmp_path / "runs.py"), str(so), str(h), str(w)], cwd=root,
+                       env=dict(os.environ, PYTHONPATH=root), capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("PASS\n"), r.stdout + r.stderr
+
+
 def test_denoiser_validation(net):
     from mutracer_amd import abi
     denoise, _ = net
