@@ -662,6 +662,21 @@ constexpr int kMaxNetLayers = 19;
 
 static int pad16(int c) { return (c + 15) & ~15; }
 
+// What repeated runs set up for their host copies, shared by the denoisers of a
+// device and given back with the last of them (host copies, below).
+struct HostPath {
+  std::mutex m;  // held while the streams are made and while `result` is in use
+  hipStream_t s[2] = {nullptr, nullptr};
+  HostBuf result;
+  HostPath() = default;
+  HostPath(const HostPath &) = delete;
+  HostPath &operator=(const HostPath &) = delete;
+  ~HostPath() {
+    for (hipStream_t c : s)
+      if (c) (void)hipStreamDestroy(c);
+  }
+};
+
 struct DenoiserObj {
   bool bf16 = false;
   bool large = false;
@@ -687,12 +702,11 @@ struct DenoiserObj {
   // Prefilters of the albedo and normal guides (clean-auxiliary models).
   std::shared_ptr<DenoiserObj> auxAlbedo, auxNormal;
   hipStream_t stream = nullptr;
-  HostBuf result;                              // on its way to the caller
-  hipStream_t copies[2] = {nullptr, nullptr};  // beside `stream` for large uploads, made by the first
+  uint32_t runs = 0;
+  HostBuf result;                  // of the first runs, on its way to the caller
+  std::shared_ptr<HostPath> path;  // of the later ones
   std::mutex busy;
   ~DenoiserObj() {
-    for (hipStream_t c : copies)
-      if (c) (void)hipStreamDestroy(c);
     if (stream) (void)hipStreamDestroy(stream);
   }
 };
@@ -927,14 +941,28 @@ static void download_layer(DenoiserObj &D, int i, int H, int W, float *out, hipS
 }
 
 // Host copies of a run. Its images come from and go to pageable memory, and a
-// copy of that goes at the pace of the thread that issues it, so large images
-// go up on three threads, each with a stream (blocking streams, ordered after
-// earlier null-stream work as D.stream is). The result passes through pinned
-// memory of the denoiser's own and is copied to the caller's buffer once it is
-// whole: a run that fails leaves the caller's buffer as it was (1080p 4.4 ms a
-// run with parts of the result straight into that buffer, 4.6 so).
-constexpr size_t kThreadedUploadBytes = 4u << 20;  // 509 x 287 (7 MB in): 0.73 -> 0.64 ms; small runs need no threads
-constexpr size_t kThreadedCopyBytes = 4u << 20;    // results that threads copy to the caller
+// copy of that goes at the pace of the thread that issues it.
+//   - The result passes through memory of the library's own and is copied to
+//     the caller's buffer once it is whole: a run that fails leaves the
+//     caller's buffer as it was.
+//   - From run kRepeated on that memory is pinned, and large images go up on
+//     three threads, each with a stream (blocking streams, ordered after
+//     earlier null-stream work as D.stream is); from the first run on where
+//     another denoiser has set these up.
+// Not earlier, because two more streams and 33 MB of pinned memory take 13 to
+// 16 ms when they are a process's first, and save 1 to 2.5 ms a run. ms of the
+// first, the second, the next and (here) the ninth and later runs of a process:
+//                                             1920 x 1080         509 x 287
+//   one stream, result through a new vector   27.0 13.7 13.5      11.2 2.7 1.1
+//   streams at once, result in place          30.3  5.0  4.4      21.6 2.6 0.61
+//   here                                      26.9  7.8  7.2 4.5  11.2 2.4 0.74 0.60
+// and of a new denoiser's first run beside others 14.2, 7.6 and 8.4 (1920 x
+// 1080), 1.28, 1.34 and 1.12 (509 x 287).
+constexpr uint32_t kRepeated = 8;
+// Inputs that go up on threads: 1280 x 720 (44 MB in) 3.4 -> 2.2 ms a run; at
+// 509 x 287 (7 MB) the streams' set-up is 10 ms for 0.05 ms a run.
+constexpr size_t kThreadedUploadBytes = 32u << 20;
+constexpr size_t kThreadedCopyBytes = 4u << 20;  // results that threads copy to the caller
 
 // work(0), work(1) and work(2), on threads of their own as far as there are any to be had.
 template <class Work>
@@ -951,13 +979,36 @@ static void on_threads(const Work &work) {
   }
 }
 
+static std::mutex gHostPathsMutex;
+static std::unordered_map<int, std::weak_ptr<HostPath>> gHostPaths;
+
+// The device's host path if there is one or this run is to make it.
+static HostPath *host_path(DenoiserObj &D) {
+  if (D.path) return D.path.get();
+  int dev = 0;
+  MTX_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> g(gHostPathsMutex);
+  std::weak_ptr<HostPath> &known = gHostPaths[dev];
+  D.path = known.lock();
+  if (!D.path && D.runs >= kRepeated) known = D.path = std::make_shared<HostPath>();
+  if (D.path) D.result.release();
+  return D.path.get();
+}
+
+// Whether both of the path's streams are there, or can be made in this run.
+static bool upload_streams(HostPath &P, bool make) {
+  std::lock_guard<std::mutex> g(P.m);
+  for (hipStream_t &s : P.s)
+    if (!s && (!make || hipStreamCreate(&s) != hipSuccess)) {
+      (void)hipGetLastError();
+      return false;
+    }
+  return true;
+}
+
 static void upload_images(DenoiserObj &D, const float *const (&src)[3], size_t bytes) {
-  bool threads = 3 * bytes >= kThreadedUploadBytes;
-  for (hipStream_t &s : D.copies) {
-    if (!threads || s) continue;
-    threads = hipStreamCreate(&s) == hipSuccess;
-    if (!threads) (void)hipGetLastError();
-  }
+  HostPath *P = host_path(D);
+  const bool threads = P && 3 * bytes >= kThreadedUploadBytes && upload_streams(*P, D.runs >= kRepeated);
   if (!threads) {
     for (int k = 0; k < 3; k++)
       MTX_HIP(hipMemcpyAsync(D.io[k].ptr, src[k], bytes, hipMemcpyHostToDevice, D.stream));
@@ -967,7 +1018,7 @@ static void upload_images(DenoiserObj &D, const float *const (&src)[3], size_t b
   MTX_HIP(hipGetDevice(&dev));
   hipError_t err[3] = {hipSuccess, hipSuccess, hipSuccess};
   on_threads([&](int k) {
-    const hipStream_t s = k ? D.copies[k - 1] : D.stream;
+    const hipStream_t s = k ? P->s[k - 1] : D.stream;
     err[k] = hipSetDevice(dev);
     if (err[k] == hipSuccess) err[k] = hipMemcpyAsync(D.io[k].ptr, src[k], bytes, hipMemcpyHostToDevice, s);
     if (err[k] == hipSuccess) err[k] = hipStreamSynchronize(s);
@@ -976,7 +1027,10 @@ static void upload_images(DenoiserObj &D, const float *const (&src)[3], size_t b
 }
 
 static void download_result(DenoiserObj &D, float *out, size_t bytes) {
-  char *const from = static_cast<char *>(D.result.ensure(bytes, true));
+  HostPath *P = host_path(D);
+  std::unique_lock<std::mutex> lk;
+  if (P) lk = std::unique_lock<std::mutex>(P->m);
+  char *const from = static_cast<char *>(P ? P->result.ensure(bytes, true) : D.result.ensure(bytes, false));
   MTX_HIP(hipMemcpyAsync(from, D.io[3].ptr, bytes, hipMemcpyDeviceToHost, D.stream));
   MTX_HIP(hipStreamSynchronize(D.stream));
   if (bytes < kThreadedCopyBytes) {
@@ -1229,6 +1283,7 @@ int32_t mtx_denoiser_run(mtx_handle handle, uint32_t width, uint32_t height, con
                   D->io[3].ptr, s);
     MTX_HIP(hipGetLastError());
     download_result(*D, output, bytes);
+    D->runs++;
     return MTX_OK;
   } catch (const Error &e) {
     set_error(err, cap, e.what());

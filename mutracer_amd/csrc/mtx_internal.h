@@ -81,7 +81,7 @@ struct DevBuf {
   }
 };
 
-// Owning host memory, pinned if asked for and to be had.
+// Owning host memory, pinned where that is asked for and to be had.
 struct HostBuf {
   void *ptr = nullptr;
   size_t bytes = 0;
@@ -90,9 +90,9 @@ struct HostBuf {
   HostBuf(const HostBuf &) = delete;
   HostBuf &operator=(const HostBuf &) = delete;
   ~HostBuf() { release(); }
-  // At least n bytes; what it held before is lost if it has to grow or change.
+  // At least n bytes; what it held before is lost when it grows.
   void *ensure(size_t n, bool pin) {
-    if (bytes >= n && (pinned || !pin)) return ptr;
+    if (bytes >= n) return ptr;
     release();
     if (pin) {
       pinned = hipHostMalloc(&ptr, n, 0) == hipSuccess;

@@ -291,12 +291,13 @@ def test_tiles(net):
     assert _rel(out[..., :3], ref[..., :3]) <= RUN_TOL["fp16"]
 
 
-@pytest.mark.parametrize("h,w", [(273, 320), (274, 320)])
+# Results below and from 4 MiB on (three threads copy them to the caller, in
+# unequal thirds), inputs below and from 32 MiB on (three threads upload them).
+@pytest.mark.parametrize("h,w", [(273, 320), (511, 512), (513, 512), (819, 853), (819, 854)])
 def test_run_host_copies(net, h, w):
-    """Images on both sides of the size from which a run's host copies go out
-    on threads (4 MiB of inputs, 87381 pixels; 274 x 320 has a download of
-    unequal thirds): tiled runs equal the untiled runs of their regions,
-    which are below that size, stitched bit for bit, twice."""
+    """A denoiser's first runs and its later ones, which use pinned memory and
+    threaded uploads (from the ninth on): tiled runs equal the untiled runs
+    of their regions, stitched bit for bit."""
     denoise, _ = net
     d = denoise.Denoiser("fp16")
     d.set_input_scale(0.8)
@@ -309,25 +310,43 @@ def test_run_host_copies(net, h, w):
             y0, y1, x0, x1 = max(0, ty - ov), min(h, ty + t + ov), max(0, tx - ov), min(w, tx + t + ov)
             r = d.run(*[np.ascontiguousarray(a[y0:y1, x0:x1]) for a in images])
             expect[ty:ty + t, tx:tx + t] = r[ty - y0:ty - y0 + t, tx - x0:tx - x0 + t]
+    d = denoise.Denoiser("fp16")
+    d.set_input_scale(0.8)
     d.set_tiles(t, ov)
-    for _ in range(2):
+    for _ in range(11):
         out = d.run(*images)
         assert np.array_equal(out, expect)
         assert np.array_equal(out[..., 3], images[0][..., 3])
+    small = [np.ascontiguousarray(a[:64, :48]) for a in images]
+    plain = denoise.Denoiser("fp16")
+    plain.set_input_scale(0.8)
+    assert np.array_equal(d.run(*small), plain.run(*small))  # buffers larger than the image
 
 
-# A hipMemcpyAsync that can be told to refuse one copy from the device.
-REFUSE = """
+# Stand-ins for calls of the runtime: a copy that can be told to refuse one from
+# the device, and counts of what takes milliseconds to set up.
+RUNTIME = """
 #include <stddef.h>
 #include <dlfcn.h>
 typedef int (*copy_fn)(void *, const void *, size_t, int, void *);
+typedef int (*stream_fn)(void **);
+typedef int (*pinned_fn)(void **, size_t, unsigned);
 static copy_fn next;
-static int left;
-int refuse_from(const char *runtime) {
+static stream_fn next_stream;
+static pinned_fn next_pinned;
+static int left, streams, pinned;
+int from_runtime(const char *runtime) {
   void *h = dlopen(runtime, RTLD_NOW | RTLD_NOLOAD);
-  next = h ? (copy_fn)dlsym(h, "hipMemcpyAsync") : 0;
-  return next != 0;
+  if (!h) return 0;
+  next = (copy_fn)dlsym(h, "hipMemcpyAsync");
+  next_stream = (stream_fn)dlsym(h, "hipStreamCreate");
+  next_pinned = (pinned_fn)dlsym(h, "hipHostMalloc");
+  return next && next_stream && next_pinned;
 }
+int streams_made(void) { return streams; }
+int pinned_made(void) { return pinned; }
+int hipStreamCreate(void **s) { streams++; return next_stream(s); }
+int hipHostMalloc(void **p, size_t n, unsigned flags) { pinned++; return next_pinned(p, n, flags); }
 void refuse(int nth) { left = nth; }
 int refused(void) { return left == 0; }
 int hipMemcpyAsync(void *dst, const void *src, size_t n, int kind, void *stream) {
@@ -335,18 +354,20 @@ int hipMemcpyAsync(void *dst, const void *src, size_t n, int kind, void *stream)
   return next(dst, src, n, kind, stream);
 }
 """
-FAILED_RUNS = """
+RUNTIME_SETUP = """
 import ctypes as C, sys
 lib = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)  # before the runtime: the library's calls go through it
 import numpy as np
 from mutracer_amd import abi, denoise
 abi.lib()
 runtime = {l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l}
-assert len(runtime) == 1 and lib.refuse_from(runtime.pop().encode())
+assert len(runtime) == 1 and lib.from_runtime(runtime.pop().encode())
 h, w = int(sys.argv[2]), int(sys.argv[3])
 rng = np.random.default_rng(3)
 im = [rng.random((h, w, 4), np.float32) for _ in range(3)]
 d = denoise.Denoiser("fp16")
+"""
+FAILED_RUNS = """
 want = d.run(*im)
 P = lambda a: a.ctypes.data_as(C.c_void_p)
 failures = 0
@@ -369,23 +390,55 @@ print("PASS")
 """
 
 
+SETUP_OF_RUNS = """
+made = lib.streams_made(), lib.pinned_made()
+first = d.run(*im)
+for run in range(1, 8):
+    assert np.array_equal(d.run(*im), first)
+    assert (lib.streams_made(), lib.pinned_made()) == made, run
+for run in range(4):
+    assert np.array_equal(d.run(*im), first)
+large = 3 * im[0].nbytes >= 32 << 20
+assert (lib.streams_made(), lib.pinned_made()) == (made[0] + (2 if large else 0), made[1] + 1)
+made = lib.streams_made()
+other = denoise.Denoiser("fp16")
+assert lib.streams_made() == made + 1  # its own
+del d  # its streams go on being the other's
+assert np.array_equal(other.run(*im), first) and np.array_equal(other.run(*im), first)
+assert lib.streams_made() == made + 1
+print("PASS")
+"""
+
+
+def _in_own_process(tmp_path, program, h, w):
+    import subprocess
+    import sys
+    (tmp_path / "runtime.c").write_text(RUNTIME)
+    (tmp_path / "runs.py").write_text(RUNTIME_SETUP + program)
+    so = tmp_path / "runtime.so"
+    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", str(tmp_path / "runtime.c"), "-o", str(so), "-ldl"],
+                   check=True)
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, str(tmp_path / "runs.py"), str(so), str(h), str(w)], cwd=root,
+                       env=dict(os.environ, PYTHONPATH=root), capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and r.stdout.endswith("PASS\n"), r.stdout + r.stderr
+
+
 @pytest.mark.parametrize("h,w", [(64, 80), (287, 509), (819, 854)])
 def test_failed_download_leaves_the_output(net, tmp_path, h, w):
     """A run whose copy of the result from the device is refused (by a
     stand-in for the runtime's copy call, in a process of its own) fails and
     leaves the caller's buffer as it was, in first and in later runs; the
     runs after it give the result."""
-    import subprocess
-    import sys
-    (tmp_path / "refuse.c").write_text(REFUSE)
-    (tmp_path / "runs.py").write_text(FAILED_RUNS)
-    so = tmp_path / "refuse.so"
-    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", str(tmp_path / "refuse.c"), "-o", str(so), "-ldl"],
-                   check=True)
-    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-    r = subprocess.run([sys.executable, str(tmp_path / "runs.py"), str(so), str(h), str(w)], cwd=root,
-                       env=dict(os.environ, PYTHONPATH=root), capture_output=True, text=True, timeout=100)
-    assert r.returncode == 0 and r.stdout.endswith("PASS\n"), r.stdout + r.stderr
+    _in_own_process(tmp_path, FAILED_RUNS, h, w)
+
+
+@pytest.mark.parametrize("h,w", [(287, 509), (819, 853), (819, 854)])
+def test_first_runs_set_nothing_up(net, tmp_path, h, w):
+    """Streams and pinned memory, which take milliseconds when they are a
+    process's first, are made in a denoiser's ninth run and once; a few runs
+    do not pay for them."""
+    _in_own_process(tmp_path, SETUP_OF_RUNS, h, w)
 
 
 def test_denoiser_validation(net):
