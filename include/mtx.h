@@ -429,7 +429,9 @@ int32_t mtx_target_synchronize(mtx_handle target);
 /* Resolved RGBA f32, top row first (Render.readPixels, Render.ts:782-801),
  * normalized as the output pass does (WGPURayTraceOutput.ts:32-92,
  * hdr_resolve_component in compose.frag.wgsl.ts:264-272); pixels without
- * samples are 0. pixels == NULL queries the float count through *written. */
+ * samples are 0. pixels == NULL queries the float count through *written.
+ * Resolves on the device into 16 bytes per pixel, which the target keeps for
+ * its next call up to 64 MiB. */
 int32_t mtx_target_read_pixels(mtx_handle target, uint32_t kind, float *pixels, size_t capacity_floats,
                                size_t *written);
 
@@ -712,6 +714,8 @@ int32_t mtx_server_submit(mtx_handle server, mtx_handle scene, const mtx_target_
  * this round; *idle = 1 when there was nothing to run. */
 int32_t mtx_server_step(mtx_handle server, void *stream, uint32_t *completed, uint32_t *idle);
 int32_t mtx_server_job_info(mtx_handle server, mtx_handle job, mtx_served_job_info *info);
+/* mtx_target_read_pixels of a job; the server keeps the same 64 MiB at most,
+ * which are not part of the HBM budget. */
 int32_t mtx_server_job_read_pixels(mtx_handle server, mtx_handle job, uint32_t kind, float *pixels,
                                    size_t capacity_floats, size_t *written);
 int32_t mtx_server_job_read_accumulators(mtx_handle server, mtx_handle job, double *sums, size_t capacity_doubles,

@@ -644,8 +644,9 @@ __global__ void __launch_bounds__(256) k_resolve(const double *__restrict__ pl, 
   }
   pixels[(size_t)(H - 1 - y) * W + x] = make_float4((float)r[0], (float)r[1], (float)r[2], (float)r[3]);
 }
-// The resolved image into host memory, through `work` (kept by the caller,
-// which serializes the calls that share it).
+// The resolved image into host memory, through `work` (kept by the caller up
+// to kResolvedKept bytes; it serializes the calls that share it).
+constexpr size_t kResolvedKept = 64u << 20;  // 4M pixels
 static void resolve_pixels(const double *planes, const uint32_t *count, uint32_t W, uint32_t H, uint32_t kind,
                            DevBuf<float4> &work, float *pixels, hipStream_t s) {
   const size_t N = (size_t)W * H;
@@ -655,6 +656,7 @@ static void resolve_pixels(const double *planes, const uint32_t *count, uint32_t
   MTX_HIP(hipGetLastError());
   work.download(reinterpret_cast<float4 *>(pixels), N, s);
   MTX_HIP(hipStreamSynchronize(s));
+  if (work.bytes() > kResolvedKept) work.release();
 }
 
 // Pixel-major copy of the 13 planes (13 doubles per pixel).

@@ -383,6 +383,22 @@ def test_read_pixels_kinds(env, w, h):
         assert np.array_equal(t.read_pixels(kind), e.astype(np.float32)), kind
 
 
+@pytest.mark.parametrize("h,kept", [(2048, 64), (2049, 0)])
+def test_read_pixels_keeps_at_most_64_mib(env, h, kept):
+    """The device image of read_pixels stays for the next call up to 2048 x
+    2048 pixels; a larger one is given back."""
+    torch, render, scene = env
+    rs = render.RenderScene(scene.cornell_box())
+    small = render.RenderTarget(rs, 8, 8, bounces=1)
+    small.read_pixels()  # the kernel's code is loaded
+    t = render.RenderTarget(rs, 2048, h, bounces=1)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for kind in ("color", "albedo"):
+        assert not t.read_pixels(kind).any()
+        assert abs((free - torch.cuda.mem_get_info()[0]) / 2**20 - kept) <= 4
+
+
 @pytest.mark.parametrize("tuning", [
     dict(trace_kernel=0, lds_stack=16),
     dict(trace_kernel=1, lds_stack=16),

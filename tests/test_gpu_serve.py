@@ -99,6 +99,22 @@ def test_job_matches_oracle(env, orc):
     assert server.info(other)["state"] == "complete"
 
 
+def test_read_pixels_memory_of_a_server(env):
+    """A server gives the device image of a large job's read_pixels back."""
+    import torch
+    render, serve, scenes, rs = env
+    server = serve.Server()
+    small = server.submit(rs[0], 32, 20, 1, bounces=1)
+    big = server.submit(rs[0], 2048, 2056, 1, bounces=1)
+    _serve_all(server, rs, [])
+    server.read_pixels(small)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    image = server.read_pixels(big)
+    assert image.shape == (2056, 2048, 4) and (free - torch.cuda.mem_get_info()[0]) >> 20 <= 4
+    assert np.array_equal(server.read_pixels(big), image)
+
+
 def test_admission_budget_and_release(env):
     render, serve, scenes, rs = env
     one_job = 40 * 30 * (13 * 8 + 4)
