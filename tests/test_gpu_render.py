@@ -383,6 +383,31 @@ def test_read_pixels_kinds(env, w, h):
         assert np.array_equal(t.read_pixels(kind), e.astype(np.float32)), kind
 
 
+def test_read_pixels_of_partly_sampled_images(env):
+    """Pixels with fewer samples than others and with none: per-pixel sample
+    targets of 0 to 3 (zero resolves to 0; the variance's alpha is 1)."""
+    torch, render, scene = env
+    w, h = 61, 37
+    t = render.RenderTarget(render.RenderScene(scene.cornell_box()), w, h, bounces=3, max_samples=3)
+    targets = np.random.default_rng(4).integers(0, 4, (h, w)).astype(np.float32)
+    t.set_sample_targets(targets)
+    t.render(3)
+    sums, counts = t.read_accumulators()
+    assert np.array_equal(counts, targets.astype(counts.dtype)) and len(np.unique(counts)) == 4
+    none = (counts == 0)[::-1]
+    sums, n = sums[::-1], np.maximum(counts[::-1], 1).astype(np.float64)
+    color = sums[..., 0:4] / np.maximum(sums[..., 11:12], 1.0)
+    hit = sums[..., 7]
+    color[..., 0:3] = np.where(hit[..., None] > 0, sums[..., 0:3] / np.where(hit > 0, hit, 1.0)[..., None], color[..., 0:3])
+    lum = (0.2126 * sums[..., 0] + 0.7152 * sums[..., 1] + 0.0722 * sums[..., 2]) / n
+    var = np.maximum(0.0, sums[..., 12] / n - lum * lum) / n
+    got = {k: t.read_pixels(k) for k in ("color", "albedo", "normal", "variance")}
+    assert np.array_equal(got["color"], color.astype(np.float32))
+    assert np.array_equal(got["variance"][..., 0], var.astype(np.float32)) and np.all(got["variance"][..., 3] == 1)
+    for k in ("color", "albedo", "normal"):
+        assert np.all(got[k][none] == 0) and np.any(got[k][~none] != 0), k
+
+
 @pytest.mark.parametrize("h,kept", [(2048, 64), (2049, 0)])
 def test_read_pixels_keeps_at_most_64_mib(env, h, kept):
     """The device image of read_pixels stays for the next call up to 2048 x
