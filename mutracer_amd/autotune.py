@@ -6,19 +6,25 @@ the knobs are the wavefront kernels' launch shape (mtx_wavefront_tuning):
 LDS stack depth, grid oversubscription, the shade kernel's
 occupancy target, the queue length below which the tail kernel finishes a
 generation, and the number of paths in flight. The tuner measures each
-candidate with HIP events (RenderTarget.render_timed) on a short probe
-render of the real target and keeps the fastest, searching one dimension at
-a time (coordinate descent, two passes). Every candidate renders the same
-samples, so tuning never changes an image; probes restart the target's
-accumulation, which the caller resets anyway before a real render.
+candidate on a short probe render of the real target, launched as any other
+render is (RenderTarget.render_timed takes the launches apart and replays no
+graph), and keeps the fastest, searching one dimension at a time (coordinate
+descent, two passes). Every candidate renders the same samples, so tuning
+never changes an image; probes restart the target's accumulation, which the
+caller resets anyway before a real render.
 
-Results are cached per (device, scene size, resolution, bounces, candidates)
-in a JSON file so a server or a repeated render tunes once.
+Results are cached per (launch form, device, scene size, resolution, bounces,
+candidates) in a JSON file so a server or a repeated render tunes once.
 """
 from __future__ import annotations
 
 import json
 import os
+import time
+
+# Raised when the kernels or their launch sequence change: what was tuned for
+# earlier ones is not applied.
+LAUNCH_FORM = 2
 
 SPACE = {
     "lds_stack": [16, 24, 32],
@@ -28,10 +34,9 @@ SPACE = {
     "max_paths_in_flight": [1 << 23, 1 << 24, 1 << 25],
     "tail_paths": [0, 16384, 65536, 262144],
     "queue_sort": [0, 1],
-    "lds_stack_closest": [0, 16, 24, 32],  # 0: the any-hit depth (lds_stack)
 }
 ORDER = ["max_paths_in_flight", "tail_paths", "queue_sort", "trace_oversubscription",
-         "shade_waves_per_simd", "shade_oversubscription", "lds_stack", "lds_stack_closest"]
+         "shade_waves_per_simd", "shade_oversubscription", "lds_stack"]
 
 
 def _key(target):
@@ -43,17 +48,23 @@ def _key(target):
     s = target.settings
     tris = target.scene.info()["triangles"]
     bucket = 1 << max(0, int(tris).bit_length() - 1)
-    return f"{name.value.decode()}|{cus.value}|tris~{bucket}|{s.width}x{s.height}|b{s.bounces}|c{s.direct_light_candidates}"
+    return f"form{LAUNCH_FORM}|{name.value.decode()}|{cus.value}|tris~{bucket}|{s.width}x{s.height}|b{s.bounces}|c{s.direct_light_candidates}"
 
 
-def probe(target, tuning, samples):
-    """GPU milliseconds of one probe render with `tuning` (after one warm-up)."""
+def probe(target, tuning, samples, repeats=3):
+    """Milliseconds of one probe render with `tuning`, the least of `repeats`
+    (after one that records the launches)."""
     target.set_tuning(**tuning)
-    target.restart_samples()
-    target.render_timed(1)
-    target.restart_samples()
-    t = target.render_timed(samples)
-    return t["generate_accumulate"] + t["trace"] + t["shade"] + t["shadow"] + t["tail"]
+    best = float("inf")
+    for k in range(repeats + 1):
+        target.restart_samples()
+        target.synchronize()
+        t0 = time.perf_counter()
+        target.render(samples)
+        target.synchronize()
+        if k:
+            best = min(best, (time.perf_counter() - t0) * 1e3)
+    return best
 
 
 def tune(target, samples=2, cache_path=None, log=None):
@@ -70,6 +81,8 @@ def tune(target, samples=2, cache_path=None, log=None):
         target.set_tuning(**cache[key]["tuning"])
         return cache[key]["tuning"]
     best = target.tuning()
+    # One kernel runs both kinds of queries, with the larger of the two depths.
+    best.update(lds_stack=max(best["lds_stack"], best["lds_stack_closest"]), lds_stack_closest=0)
     best_ms = probe(target, best, samples)
     trials = [(dict(best), best_ms)]
     for _ in range(2):

@@ -501,6 +501,16 @@ def test_autotune(env, orc, tmp_path):
     assert np.array_equal(t.read_accumulators()[0], ref)
 
 
+def test_autotune_measures_replayed_graphs(env):
+    torch, render, scene = env
+    from mutracer_amd import autotune
+    t = render.RenderTarget(render.RenderScene(scene.cornell_box()), 32, 24, bounces=3, max_samples=2)
+    before = t.tuning()
+    assert autotune.probe(t, before, 2) > 0.0
+    after = t.tuning()
+    assert after["graph_captures"] == 1 and after["graph_replays"] >= 4
+
+
 @pytest.mark.parametrize("kernel", KERNELS)
 def test_adaptive_converge(env, orc, kernel):
     """Pilot moments -> per-tile plan (the reference formula, recomputed here
