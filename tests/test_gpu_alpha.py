@@ -10,7 +10,8 @@ that camera and secondary rays pass through them. Both sides restate the
 same rules (coverage resolution, pass-through vertex without a depth,
 shadow-ray coverage test), so the FP64 accumulators agree bit for bit on
 both kernel forms, every sampling pattern and every wavefront launch form
-(stack or persistent walker traversal, tail kernel, queue sorting).
+(shadow rays in the next event's launch or in their own, tail kernel, queue
+sorting, several jobs in one round).
 """
 import numpy as np
 import pytest
@@ -63,10 +64,31 @@ def test_panes_match_oracle(env, orc, kernel, pattern, panes):
     assert np.array_equal(got, ref)
 
 
+@pytest.mark.parametrize("large", [False, True])
+def test_masked_jobs_in_one_round_match_oracle(env, orc, large):
+    """Masked and opaque scenes share a server's rounds: the coverage test
+    finds each shadow ray's own scene, with the tail kernel (small scenes
+    only) and with shadow rays in the next event's launch (a large one among
+    them)."""
+    abi, render, scene = env
+    from mutracer_amd import serve
+    scenes = [scene.alpha_caster("checker"), scene.masked_panes(2, checker=True), scene.cornell_box()]
+    if large:
+        scenes.append(scene.instanced_field(n_instances=6, freq=8, env_size=(64, 32)))
+    server = serve.Server(max_samples_per_job_round=2)
+    jobs = [(sc, 40 + 3 * k, 30 - k, server.submit(render.RenderScene(sc), 40 + 3 * k, 30 - k, 4, bounces=5,
+                                                   direct_light_candidates=2)) for k, sc in enumerate(scenes)]
+    while not server.step()[1]:
+        pass
+    for sc, w, h, job in jobs:
+        ref = orc.OracleRenderer(sc, w, h, bounces=5, candidates=2, max_samples=4).render(0, 4)
+        assert np.array_equal(server.read_accumulators(job)[0], ref)
+
+
 @pytest.mark.parametrize("tuning", [
-    dict(trace_kernel=0, tail_paths=0),
-    dict(trace_kernel=1, tail_paths=0),
-    dict(trace_kernel=1, tail_paths=600),
+    dict(tail_paths=0),
+    dict(lds_stack=32, use_graphs=0, tail_paths=0),
+    dict(tail_paths=600),
     dict(tail_paths=1 << 30),
     dict(queue_sort=1, tail_paths=0),
 ])

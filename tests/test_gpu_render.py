@@ -425,16 +425,16 @@ def test_read_pixels_keeps_at_most_64_mib(env, h, kept):
 
 
 @pytest.mark.parametrize("tuning", [
-    dict(trace_kernel=0, lds_stack=16),
-    dict(trace_kernel=1, lds_stack=16),
-    dict(trace_kernel=1, lds_stack=24, trace_oversubscription=2),
-    dict(trace_kernel=1, lds_stack=32, shade_oversubscription=3, max_paths_in_flight=3000),
-    dict(trace_kernel=0, shade_waves_per_simd=2),
-    dict(trace_kernel=0, shade_waves_per_simd=4, shade_oversubscription=2),
+    dict(lds_stack=16),
+    dict(trace_kernel=1, use_graphs=0),
+    dict(lds_stack=24, trace_oversubscription=2),
+    dict(lds_stack=32, shade_oversubscription=3, max_paths_in_flight=3000),
+    dict(shade_waves_per_simd=2),
+    dict(shade_waves_per_simd=4, shade_oversubscription=2),
     dict(tail_paths=0),
     dict(tail_paths=1500),
     dict(tail_paths=1 << 30),
-    dict(trace_kernel=1, tail_paths=3000, max_paths_in_flight=9000),
+    dict(use_graphs=0, tail_paths=3000, max_paths_in_flight=9000),
     dict(lds_stack_closest=16),
     dict(lds_stack_closest=32, lds_stack=24),
     dict(queue_sort=1),
