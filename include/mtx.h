@@ -446,7 +446,7 @@ int32_t mtx_target_read_accumulators(mtx_handle target, double *sums, size_t cap
 typedef struct mtx_wavefront_tuning {
   uint32_t struct_size;
   uint32_t max_paths_in_flight;    /* paths per generation (0 = keep) */
-  uint32_t trace_kernel;           /* 0 or 1; both run the wave-scheduled traversal kernels */
+  uint32_t trace_kernel;           /* deprecated: 0 or 1, kept for get and otherwise ignored */
   uint32_t lds_stack;              /* traversal LDS stack entries per lane: 16, 24 or 32 */
   uint32_t trace_oversubscription; /* trace grid = CUs x resident blocks x this (>= 1) */
   uint32_t shade_oversubscription; /* shade grid likewise (>= 1) */

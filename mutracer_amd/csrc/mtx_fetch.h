@@ -24,8 +24,9 @@ constexpr int kXcds = 8;
 // Occupancy the register allocator must reach for the traversal kernels
 // (waves per SIMD): 5 (96 VGPRs) for the wavefront kernels and closest-hit
 // queries, where 6 spills (closest hit of the 1M-triangle 1080p step 66.5 ms
-// against 50.2, 4 waves 62 ms; shadow rays 26.1 against 25.8), 6 (no spill)
-// for the smaller any-hit query (1.01 ms against 1.04 for 1.5M rays).
+// against 50.2, 4 waves 62 ms; shadow rays 26.1 against 25.8; each in a kernel
+// of its own), 6 (no spill) for the smaller any-hit query (1.01 ms against 1.04
+// for 1.5M rays).
 constexpr int kTraceWaves = 5;
 constexpr int kOcclusionWaves = 6;
 

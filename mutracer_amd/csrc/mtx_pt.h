@@ -180,9 +180,9 @@ struct WfConfig {
   uint32_t maxPaths = 1u << 25;  // paths in flight per generation
   int traceOversub = 1;          // trace/shadow grid = CUs * resident blocks * this
   int shadeOversub = 1;
-  uint32_t traceKernel = 0;      // mtx_wavefront_tuning.trace_kernel as set; both values run the same kernels
-  int ldsStack = 16;             // LDS stack entries per lane of the any-hit kernels (16, 24 or 32)
-  int ldsStackClosest = 0;       // the same for the closest-hit trace kernel (0 = ldsStack)
+  uint32_t traceKernel = 0;      // mtx_wavefront_tuning.trace_kernel as set (ignored)
+  int ldsStack = 16;             // LDS stack entries per lane of the query kernel (16, 24 or 32)
+  int ldsStackClosest = 0;       // the same as asked for closest hits (0 = ldsStack); the larger counts
   int shadeWaves = 2;            // occupancy target of the shade kernel (1..4 waves per SIMD)
   bool graphs = true;            // capture each generation's launch sequence into a hipGraph and replay it
   uint32_t tailPaths = 0;        // the tail kernel finishes the paths once a queue is this short (0 = never);

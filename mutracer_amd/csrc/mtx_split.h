@@ -12,7 +12,12 @@ constexpr uint32_t queue_lanes(uint32_t n, uint32_t waves) {
   return per < 1u ? 1u : (per > 64u ? 64u : (uint32_t)per);
 }
 
-// Entries of a chunk: one per lane, up to four in queues of thousands a wave.
+// Entries of a chunk: one per lane, and up to four per lane where a wave takes
+// more than 512 entries, so that a wave keeps to neighbouring rays. 1M-triangle
+// 1080p step: 133.9 ms, with at most one per lane 136.7, sixteen 134.5, from
+// 128 entries a wave on 134.7, from 2048 on 135.0. 16M camera rays in 24 x 60k
+// triangles: 3.43, 3.95, 3.68, 3.42, 3.93 ms; 6M in 1M triangles 2.09, 2.21,
+// 2.09, 2.21, 2.22; 4M scattered rays 9.18, 9.18, 9.18, 9.64, 9.18.
 constexpr uint32_t queue_chunk(uint32_t n, uint32_t waves) {
   const uint32_t lanes = queue_lanes(n, waves);
   if (lanes < 64u) return lanes;

@@ -10,17 +10,20 @@
 // all three bodies per iteration with a few lanes each (22% of the lanes of an
 // instruction were active). Here the wave counts its lanes, runs the body that
 // most of them wait for and lets the others wait, and takes new rays for the
-// lanes that have finished once enough of them have (37% active).
+// lanes that have finished once enough of them have (36% active).
 //
 // What bounds it (1M-triangle 1080p step, closest hit): the vector memory
-// address unit is busy 78% of the cycles (about 27 cycles per 16-byte load of
-// a wave, whatever its active lanes) and the VALU issues 65% of them, both in
-// proportion to the waves' iterations. 82 -> 50 ms for its 83M closest-hit
-// rays, 49 -> 26 ms for its 53M shadow rays; 4096 rays in a 50k-triangle mesh
-// 234 -> 120 us. Fetching each node by the four lanes of a quad (16 bytes
-// each, through LDS) quarters the cache accesses but not that unit's time and
-// measured slower (56-59 ms), as did returning to the TLAS within the node
-// step (53 ms: fewer waits, more instructions in every step).
+// address unit is busy 77% of the cycles (about 27 cycles per 16-byte load of
+// a wave, whatever its active lanes) and the VALU issues 62% of them, both in
+// proportion to the waves' iterations. 82 -> 50 ms for its 80M closest-hit
+// rays, 49 -> 26 ms for its 51M shadow rays (in kernels of their own); 4096
+// rays in a 50k-triangle mesh 250 -> 104 us. Rays that share nothing are bound
+// by the caches' misses instead: 4M scattered rays in 1M triangles miss the L2
+// with 62% of their requests, some 66 GB in 9.1 ms. Fetching each node by the
+// four lanes of a quad (16 bytes each, through LDS) quarters the cache accesses
+// but not the address unit's time and measured slower (56-59 ms), as did
+// returning to the TLAS within the node step (53 ms: fewer waits, more
+// instructions in every step).
 #pragma once
 #include "mtx_accel.h"
 #include "mtx_fetch.h"
@@ -29,7 +32,8 @@ namespace mtx {
 
 // A wave keeps to interior nodes while at least kBoxEighths / 8 of its active
 // lanes are at one: 2, 3 and 4 measure 52.3, 50.8 and 50.8 ms for closest hit
-// and 27.1, 26.1 and 26.4 ms for shadow rays at the 1M-triangle 1080p step.
+// and 27.1, 26.1 and 26.4 ms for shadow rays at the 1M-triangle 1080p step
+// (each in a kernel of its own).
 constexpr int kBoxEighths = 3;
 
 // What a lane traces: filled by the kernel's load(i, ray).

@@ -12,7 +12,7 @@
 //     shade   shade_event(): emission, NEE candidate choice, BSDF sample,
 //             Russian roulette; appends the path to queue e+1 when it
 //             continues and its shadow ray to the shadow queue of event e
-//   query     the last event's shadow queue
+//             (the last event samples nothing: it has no shadow rays)
 //   accumulate each pixel's samples, in sample order, into the FP64 running
 //             sums and advance the per-pixel sample counter
 //
@@ -174,8 +174,8 @@ __device__ __forceinline__ void wave_append2(uint32_t *counts, int event, bool n
 // A wave sorts the paths it takes into bins by the shading class of what they
 // hit (LDS, a few entries per class) and shades a bin once it holds 64 paths,
 // so that its lanes run mostly the same lobes; what is left at the end is
-// shaded class by class. On the 1M-triangle 1080p step 45 -> 69% of the lanes
-// of an instruction are active and shading takes 48.6 ms instead of 64.4; the
+// shaded class by class. On the 1M-triangle 1080p step 45 -> 65% of the lanes
+// of an instruction are active and shading takes 49.3 ms instead of 64.4; the
 // loads' latency at two waves per SIMD bounds it now (the VALU issues 41% of
 // the cycles; three waves spill: 72 ms). Both queues advance with one atomic
 // per wave.
@@ -418,7 +418,10 @@ __device__ __forceinline__ void shadow_rays(const WfLaunch &L, const WfBuffers &
 // event). They are independent (a shadow ray adds to its path's radiance,
 // which no closest-hit query reads), so one launch runs both and its end is
 // the later of the two instead of their sum: a late event with a few thousand
-// rays of each kind takes one latency chain.
+// rays of each kind takes one latency chain. (For the closest hits or the
+// shadow rays alone the shared kernel takes 4 to 7% longer than one of their
+// own did, 54.0 and 27.4 ms of the 1M-triangle 1080p step against 50 and 26;
+// the shared launches take 76.8.)
 template <bool kMulti, bool kCount, int kLds, bool kAlpha>
 __global__ void __launch_bounds__(kWfTraceBlock, kTraceWaves)
 k_wf_query(const WfLaunch L, WfBuffers W, int event, int shadowEvent, int32_t *__restrict__ spill) {
