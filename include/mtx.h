@@ -159,7 +159,9 @@ typedef struct mtx_hit {
  * waves), at most about 270 MB. Queries of several threads on one stream follow one another. A closest-hit
  * or counting query recorded into a graph uses its stream's work counters on
  * every replay: no query on that stream and no graph recorded on it may run
- * beside the replay (mtx_trace_any has no counters there). */
+ * beside the replay (mtx_trace_any has no counters there). hipStreamPerThread
+ * counts as one stream for all threads; only mtx_trace_any may run on it in
+ * several at once, in scenes whose traversal stacks stay within 16 entries. */
 int32_t mtx_trace_closest(mtx_handle accel, const mtx_ray *rays, uint32_t count, mtx_hit *hits,
                           uint32_t flags, void *stream);
 

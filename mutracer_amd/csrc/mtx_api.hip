@@ -28,9 +28,10 @@ __global__ void k_zero_counters(uint32_t *__restrict__ c) {
 // Ray queries: the traversal of the wavefront trace (closest hit) and shadow
 // (any hit) kernels over a caller's rays; `ctr` holds the queue's chunk
 // counters, zeroed before the launch.
-// Mode 4 uses no counters, for queries recorded into a graph: graphs recorded
+// Mode 4 uses no counters, for queries recorded into a graph (graphs recorded
 // on one stream may be replayed on several at once, where they would share
-// that stream's counters. Outside of graphs mode 1 stays: it is 6 to 9% faster
+// that stream's counters) and on hipStreamPerThread, which is another stream
+// in each thread. Elsewhere mode 1 stays: it is 6 to 9% faster
 // where waves take many chunks (6M occlusion rays in 24 x 60k triangles 2.65 ms
 // against 2.82) and on short queries (40k 0.277 against 0.285), slower in
 // between (1.5M 0.99 against 0.92).
@@ -176,7 +177,7 @@ static void launch_trace(int mode, const Accel &A, const mtx_ray *rays, uint32_t
   if (mode == 0 && (flags & MTX_TRACE_COUNT)) mode = 3;
   // The same grid recorded or not: the scratch of a query made before suffices.
   const uint32_t grid = query_grid(n, resident_grid(mode));
-  if (mode == 1 && recording(s)) mode = 4;
+  if (mode == 1 && (s == hipStreamPerThread || recording(s))) mode = 4;
   auto S = scratch_of(s);
   std::lock_guard<std::mutex> g(S->m);
   const uint32_t waves = grid * (kTraceBlock / 64);

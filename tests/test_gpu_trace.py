@@ -238,9 +238,10 @@ def test_any_hit_recorded(orc, env, queue_scene, n):
         assert np.array_equal(got[:n].astype(np.uint32), occ[:n]) and got[n] == 7
 
 
-def test_any_hit_graphs_side_by_side(orc, env):
-    """Two occlusion queries recorded on one stream, replayed on two at once.
-    (A scene whose stacks fit in LDS: spilled ones belong to a stream.)"""
+@pytest.fixture(scope="module")
+def shallow_scene(orc, env):
+    """A scene whose traversal stacks fit in LDS (spilled ones belong to a
+    stream), rays and which of them are occluded."""
     torch, accel, W = env
     pos, idx = W.sphere_mesh(20, 10)
     scene = orc.assemble_scene([dict(positions=pos, indices=idx)],
@@ -252,7 +253,45 @@ def test_any_hit_graphs_side_by_side(orc, env):
     rays = np.zeros((50_000, 8), np.float32)
     rays[:, 0:3], rays[:, 4:7] = rng.uniform(-1.5, 1.5, (50_000, 3)), rng.normal(size=(50_000, 3))
     rays[:, 3] = rng.uniform(0.0, 2.0, 50_000)
-    occ = scene.any(rays).astype(np.int32)
+    return acc, rays, scene.any(rays).astype(np.int32)
+
+
+def test_any_hit_on_per_thread_streams(env, shallow_scene):
+    """Occlusion queries of two threads on hipStreamPerThread (handle 2)."""
+    import threading
+    import types
+    torch, accel, W = env
+    acc, rays, occ = shallow_scene
+    reps, bad = 40, []
+    dev = [torch.from_numpy(np.tile(rays[k::2], (40, 1))).cuda() for k in range(2)]
+    exp = [torch.from_numpy(np.tile(occ[k::2], 40)).cuda() for k in range(2)]
+    outs = [torch.full((reps, d.shape[0]), 7, dtype=torch.int32, device="cuda") for d in dev]
+    acc.trace_any(dev[0], outs[0][0])
+    torch.cuda.synchronize()
+
+    def ask(k):
+        try:
+            for i in range(reps):
+                acc.trace_any(dev[k], outs[k][i], stream=types.SimpleNamespace(cuda_stream=2))
+            torch.cuda.synchronize()
+        except Exception as e:
+            bad.append(e)
+
+    threads = [threading.Thread(target=ask, args=(k,)) for k in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not bad
+    for k in range(2):
+        assert bool((outs[k] == exp[k]).all())
+
+
+def test_any_hit_graphs_side_by_side(env, shallow_scene):
+    """Two occlusion queries recorded on one stream, replayed on two at once."""
+    torch, accel, W = env
+    acc, rays, occ = shallow_scene
     rec, streams, work = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()], []
     for k in range(2):
         r = torch.from_numpy(np.tile(rays[k::2], (40, 1))).cuda()
