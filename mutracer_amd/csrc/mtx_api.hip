@@ -90,6 +90,11 @@ struct StreamScratch {
   std::mutex m;
   DevBuf<int32_t> spill;
   DevBuf<uint32_t> counters;
+  std::weak_ptr<OwnStream> last;  // whose launches used `spill` last, in place of this stream's
+  hipEvent_t used = nullptr;      // their end, once another's have to wait for it
+  ~StreamScratch() {
+    if (used) (void)hipEventDestroy(used);
+  }
 };
 static std::mutex gScratchesMutex;
 static std::map<std::pair<int, hipStream_t>, std::shared_ptr<StreamScratch>> gScratches;
@@ -122,10 +127,19 @@ static int32_t *spill_of(StreamScratch &S, size_t lanes) {
   if (S.spill.count < need) S.spill = DevBuf<int32_t>(need);
   return S.spill.ptr;
 }
-int32_t *spill_for(hipStream_t s, uint32_t blocksNeeded, uint32_t blockThreads) {
-  auto S = scratch_of(s);
-  std::lock_guard<std::mutex> g(S->m);
-  return spill_of(*S, (size_t)blocksNeeded * blockThreads);
+SpillLease::SpillLease(hipStream_t s, uint32_t blocks, uint32_t blockThreads)
+    : scratch(scratch_of(s)), lock(scratch->m) {
+  ptr = spill_of(*scratch, (size_t)blocks * blockThreads);
+}
+void SpillLease::enter(const std::shared_ptr<OwnStream> &own) {
+  const auto last = scratch->last.lock();  // gone: its stream has been waited for
+  if (last && last != own && hipStreamQuery(last->s) != hipSuccess) {  // not yet done
+    (void)hipGetLastError();
+    if (!scratch->used) MTX_HIP(hipEventCreateWithFlags(&scratch->used, hipEventDisableTiming));
+    MTX_HIP(hipEventRecord(scratch->used, last->s));
+    MTX_HIP(hipStreamWaitEvent(own->s, scratch->used, 0));
+  }
+  scratch->last = own;
 }
 // Whether launches on s are being recorded into a graph.
 static bool recording(hipStream_t s) {

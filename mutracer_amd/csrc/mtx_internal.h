@@ -81,6 +81,18 @@ struct DevBuf {
   }
 };
 
+// A stream of an object's own (blocking: ordered with the null stream).
+struct OwnStream {
+  hipStream_t s = nullptr;
+  OwnStream() { MTX_HIP(hipStreamCreate(&s)); }
+  OwnStream(const OwnStream &) = delete;
+  OwnStream &operator=(const OwnStream &) = delete;
+  ~OwnStream() {
+    (void)hipStreamSynchronize(s);
+    (void)hipStreamDestroy(s);
+  }
+};
+
 // Owning host memory, pinned where that is asked for and to be had.
 struct HostBuf {
   void *ptr = nullptr;

@@ -1,6 +1,7 @@
 // Path tracer: resident render scene, render targets and kernel entry points.
 #pragma once
 #include <algorithm>
+#include <memory>
 
 #include "mtx_internal.h"
 #include "mtx_scene.h"
@@ -217,7 +218,7 @@ struct LaunchTimer {
 struct WfGraph {
   hipGraphExec_t exec = nullptr;
   uint64_t key = 0;
-  hipStream_t own = nullptr;  // capture/replay stream when the caller passes the null stream
+  std::shared_ptr<OwnStream> own;  // capture/replay stream when the caller passes the null stream
   uint64_t replays = 0, captures = 0;
   void reset();
   ~WfGraph();

@@ -127,7 +127,8 @@ void launch_render(const GpuScene &scene, const RenderParams &p, const Accumulat
   uint32_t grid = trace_grid();
   uint32_t need = ((p.pixelCount + kBlock - 1) / kBlock + 7u) / 8u * 8u;
   grid = std::min(grid, need);
-  int32_t *spill = spill_for(s, grid, kBlock);
+  const SpillLease lease(s, grid, kBlock);
+  int32_t *spill = lease.ptr;
   if (timer) timer->begin(4);
   // Shadow rays test coverage only in scenes with mask materials.
   const bool masked = (scene.features & kSceneMasked) != 0u;

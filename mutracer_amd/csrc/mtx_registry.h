@@ -36,6 +36,23 @@ struct Registry {
 
 Registry &registry();
 uint32_t trace_grid();
-int32_t *spill_for(hipStream_t s, uint32_t blocksNeeded, uint32_t blockThreads);
+
+// The spill memory of a stream's traversal stacks (ptr), held while a render
+// enqueues its launches: no other thread's launches on the stream grow (free)
+// it in between. A render whose launches run on a stream of its own in place
+// of the null stream (which cannot be recorded) calls enter() before them: the
+// memory is the null stream's, and two such streams do not follow one another
+// by themselves.
+struct StreamScratch;
+class SpillLease {
+ public:
+  SpillLease(hipStream_t s, uint32_t blocks, uint32_t blockThreads);
+  void enter(const std::shared_ptr<OwnStream> &own);
+  int32_t *ptr = nullptr;
+
+ private:
+  std::shared_ptr<StreamScratch> scratch;
+  std::unique_lock<std::mutex> lock;
+};
 
 }  // namespace mtx

@@ -692,7 +692,7 @@ void target_render(TargetObj &T, uint32_t samples, hipStream_t s, uint64_t *work
     launch_render(T.scene->view, p, acc, s, timer);
   else
     launch_render_wavefront(T.scene->view, p, acc, T.wf, T.wfConfig, s, timer, work ? nullptr : &T.graph);
-  if (!s && T.graph.own && T.kernel != MTX_KERNEL_MEGAKERNEL) s = T.graph.own;
+  if (!s && T.graph.own && T.kernel != MTX_KERNEL_MEGAKERNEL) s = T.graph.own->s;
   T.stream = s;
   T.samplesDone += samples;
 }
@@ -1303,8 +1303,8 @@ static uint32_t server_round(ServerObj &S, hipStream_t s, bool &idle) {
     // own blocking stream (ordered with the null stream's admission work).
     hipStream_t rs = s;
     if (!rs && S.cfg.graphs) {
-      if (!S.graph.own) MTX_HIP(hipStreamCreate(&S.graph.own));
-      rs = S.graph.own;
+      if (!S.graph.own) S.graph.own = std::make_shared<OwnStream>();
+      rs = S.graph.own->s;
     }
     S.cfg.tailPaths = default_tail_paths(triangles);
     S.slots.upload(slots.data(), slots.size(), rs);

@@ -814,10 +814,7 @@ void WfGraph::reset() {
   exec = nullptr;
   key = 0;
 }
-WfGraph::~WfGraph() {
-  reset();
-  if (own) (void)hipStreamDestroy(own);
-}
+WfGraph::~WfGraph() { reset(); }
 
 static uint64_t fnv(uint64_t h, const void *data, size_t n) {
   const unsigned char *b = (const unsigned char *)data;
@@ -833,7 +830,8 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
   const uint32_t maxPaths = std::max<uint32_t>(cfg.maxPaths, p0.pixelCount);
   const uint32_t genMax = std::max<uint32_t>(1u, maxPaths / p0.pixelCount);
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(g.query, g.tail), kWfTraceBlock);
+  SpillLease lease(s, std::max(g.query, g.tail), kWfTraceBlock);
+  int32_t *spill = lease.ptr;
   const int eventLimit = event_limit(scene, p0);
   uint32_t done = 0;
   while (done < p0.samples) {
@@ -860,8 +858,8 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
       // capture replays for as long as its arguments are unchanged.
       hipStream_t gs = s;
       if (!gs) {
-        if (!graph->own) MTX_HIP(hipStreamCreate(&graph->own));
-        gs = graph->own;  // blocking stream: ordered with the legacy null stream
+        if (!graph->own) graph->own = std::make_shared<OwnStream>();
+        gs = graph->own->s;  // blocking stream: ordered with the legacy null stream
       }
       uint64_t key = 1469598103934665603ull;
       static_assert(sizeof(GpuScene) == 152 && sizeof(RenderParams) % 4 == 0, "key layouts");
@@ -890,6 +888,7 @@ void launch_render_wavefront(const GpuScene &scene, const RenderParams &p0, cons
         graph->key = key;
         graph->captures++;
       }
+      if (gs != s) lease.enter(graph->own);
       MTX_HIP(hipGraphLaunch(graph->exec, gs));
       graph->replays++;
     } else {
@@ -905,7 +904,8 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
   if (!nJobs || !nPaths) return;
   MTX_REQUIRE(nJobs <= kMaxJobsPerRound, MTX_INVALID_ARGUMENT, "too many jobs in one round");
   const Grids g = grids_for(cfg);
-  int32_t *spill = spill_for(s, std::max(g.query, g.tail), kWfTraceBlock);
+  SpillLease lease(s, std::max(g.query, g.tail), kWfTraceBlock);
+  int32_t *spill = lease.ptr;
   buf.ensure(nPaths, cfg.queueSort);
   const WfBuffers W = buf.view(nPaths, cfg.queueSort);
   WfLaunch L;
@@ -922,8 +922,8 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
     // server's own blocking stream is ordered with the null stream).
     hipStream_t gs = s;
     if (!gs) {
-      if (!graph->own) MTX_HIP(hipStreamCreate(&graph->own));
-      gs = graph->own;
+      if (!graph->own) graph->own = std::make_shared<OwnStream>();
+      gs = graph->own->s;
     }
     uint64_t key = 1469598103934665603ull;
     key = fnv(key, &L, sizeof L);
@@ -946,6 +946,7 @@ void launch_generation_multi(const JobSlot *devSlots, uint32_t nJobs, uint32_t n
       graph->key = key;
       graph->captures++;
     }
+    if (gs != s) lease.enter(graph->own);
     MTX_HIP(hipGraphLaunch(graph->exec, gs));
     graph->replays++;
     return;

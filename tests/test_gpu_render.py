@@ -483,6 +483,52 @@ def test_graph_replays_match_eager(env, orc):
     assert np.array_equal(g.read_accumulators()[0], ref)
 
 
+def test_targets_rendering_side_by_side(env):
+    """Two targets whose renders are in flight together on the default stream
+    (their graphs run on streams of their own, the traversal stacks' spill
+    memory is shared), with ray queries of another thread in between, give
+    the sums each gives alone."""
+    import threading
+    torch, render, scene = env
+    from mutracer_amd import accel, workloads as W
+    scenes = [scene.instanced_field(n_instances=n, freq=f, env_size=(64, 32)) for n, f in ((20, 16), (9, 22))]
+    kw = dict(bounces=6, direct_light_candidates=2, max_samples=12)
+    targets = [render.RenderTarget(render.RenderScene(sc), 200, 120, **kw) for sc in scenes]
+    alone = []
+    for t in targets:
+        for _ in range(6):
+            t.render(2)
+        alone.append(t.read_accumulators()[0])
+        t.restart_samples()
+    pos, idx = W.random_triangles(30000, seed=3)
+    acc = accel.Accel([accel.Blas(pos, idx)], [0], [W.identity_transform()])
+    rays = torch.from_numpy(W.pinhole_rays(300)).cuda()
+    expect = torch.zeros((rays.shape[0], 8), dtype=torch.int32, device="cuda")
+    acc.trace_closest(rays, expect)
+    hits = [torch.zeros_like(expect) for _ in range(12)]
+    torch.cuda.synchronize()
+    bad = []
+
+    def ask():
+        try:
+            for h in hits:
+                acc.trace_closest(rays, h)
+        except Exception as e:
+            bad.append(e)
+
+    other = threading.Thread(target=ask)
+    other.start()
+    for _ in range(6):
+        for t in targets:
+            t.render(2)
+    other.join()
+    torch.cuda.synchronize()
+    assert not bad and all(torch.equal(h, expect) for h in hits)
+    for t, ref in zip(targets, alone):
+        sums, counts = t.read_accumulators()
+        assert np.all(counts == 12) and np.array_equal(sums, ref)
+
+
 def test_autotune(env, orc, tmp_path):
     torch, render, scene = env
     from mutracer_amd import autotune
